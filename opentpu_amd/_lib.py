@@ -17,6 +17,7 @@ INT8, INT4, FP4, NVFP4 = 0, 1, 2, 3
 FMT = {"int8": INT8, "int4": INT4, "fp4": FP4, "nvfp4": NVFP4}
 UNIT, ACC, RMAX, ASCALE, PAIR, RSC = 0x1, 0x2, 0x4, 0x8, 0x40, 0x80
 Q_ROW, Q_LO, Q_HL = 0x1, 0x10, 0x20             # QACT / QST flags
+ACT_ANY, ACT_ROW, ACT_MX = 0, 1, 2              # otpu_mm_dot: what is known of the activation offsets
 QALIGN = 64                                     # QACT ST / LDA row alignment
 LM_STATE_BYTES = 16640                          # the LM head's state (result word, maxima)
 ABI_VERSION = 3                                 # include/otpu.h OTPU_ABI_VERSION this binding follows
@@ -38,6 +39,7 @@ SIGNATURES = {
     "otpu_pack_x4": ([_P, _I, _I, _L, _I, _P, _L, _P, _L, _P], _I),
     "otpu_qact_ranges": ([_P, _P, _I, _I, _L, _I, _I, _I, _P, _P, _P, _L, _P, _P, _L, _P], _I),
     "otpu_mm_ranges": ([_P, _L, _P, _P, _L, _I, _I, _I, _P, _L, _P, _L, _I, _I, _I, _I, _P, _P, _L, _P], _I),
+    "otpu_mm_dot": ([_P, _L, _P, _P, _L, _I, _I, _I, _P, _L, _P, _L, _I, _I, _I, _I, _I, _P, _P, _L, _P], _I),
     "otpu_vmul": ([_P, _P, _P, _L, _P], _I),
     "otpu_mm_qin": ([_P, _P, _P, _P, _I, _L, _I, _I, _P, _L, _P, _L, _I, _I, _I, _I, _P, _L, _L, _P], _I),
     "otpu_mm_qin_fold": ([_P, _P, _P, _P, _I, _I, _P, _L, _P, _L, _I, _I, _I, _I, _P, _P], _I),

@@ -13,12 +13,13 @@
 // an ordinary integer matrix product of int8 activations and the integer w'' (|w''| < 2^15 when
 // the tile's offsets and multipliers allow: checked per tile).  w'' is split into two int8 planes
 // in balanced base 256 (w'' = 256 h + l, l and h in [-128, 127]), each an int8 MFMA operand, so
-// the K walk is a plain two-plane int8 GEMM with no rescaling inside it.  Activation planes (MX
-// offsets) walk K once each, combined by Horner's rule in the int32 accumulators (acc <<= the gap
-// to the next plane's d, as the int8 GEMM does; the bound is checked per tile).  The epilogue
-// forms T = 256 C_h + C_l in int64 and shifts it by W - R_n - d_last (exact: the accumulator is
-// an integer), then the reference's fp32 epilogue.  A tile the bounds refuse takes an exact VALU
-// path.
+// the K walk is a plain two-plane int8 GEMM with no rescaling inside it.  Two activation planes walk
+// K once each, combined by Horner's rule in the int32 accumulators (acc <<= the gap to the next
+// plane's d; the bound is checked per tile).  The epilogue forms T = 256 C_h + C_l in double and
+// scales it by 2^(W - R_n - d_last) (exact: the accumulator is an integer), then the reference's fp32
+// epilogue.  A tile of more offsets, or of weights past the fold's range, takes prefill_impl.h's walk
+// (at 512 x 2048 x 8192 int4 and offsets {0, 1, 2}: 89 us as three walks, 50 us so; with two offsets
+// two walks measure 51 us int4 and 57 us nvfp4, the other walk 50 and 69).
 //
 // Work layout.  A workgroup of 8 waves owns a 128 x 128 output tile.  Waves 0-3 multiply (64 x 64
 // each, 4 x 4 v_mfma_i32_16x16x64_i8 per 64-deep step and plane); waves 4-7 stream: they issue
@@ -30,7 +31,7 @@
 // barrier a stage.
 #include <type_traits>
 
-#include "otpu_common.h"
+#include "prefill_impl.h"
 
 namespace otpu {
 namespace g4 {
@@ -178,50 +179,6 @@ __device__ __forceinline__ void expand8(uint32_t x, const uint32_t (&tl)[4], con
         h0 = __builtin_amdgcn_perm(ho, he, 0x05010400u);
         h1 = __builtin_amdgcn_perm(ho, he, 0x07030602u);
     }
-}
-
-// the exact MM integer of output (j, n), group by group (the tiles the planes' bounds refuse)
-template <int FMT>
-__device__ int64_t valu_acc4(const Args& a, int j, int n, bool plainw) {
-    constexpr int mag[8] = {0, 1, 2, 3, 4, 6, 8, 12};
-    constexpr int G = Fmt<FMT>::NV ? 2 : 1, GS = 32 / G;     // weight groups a 32-group, their size
-    const int8_t* qr = a.q + (int64_t)j * a.ldq;
-    const uint8_t* wr = a.w + (int64_t)n * a.rs;
-    const uint8_t* srow = a.ws + (int64_t)n * a.srs;
-    int64_t acc = 0;
-    for (int g = 0; g < a.K / 32; ++g) {
-        const int da = (int)a.da[(int64_t)j * a.ldda + g];
-        for (int h = 0; h < G; ++h) {
-            int c = 0;
-            for (int i = GS * h; i < GS * (h + 1); ++i) {
-                const int code = (wr[16 * g + i / 2] >> (4 * (i & 1))) & 15;
-                const int v = FMT == OTPU_INT4 ? (code < 8 ? code : code - 16) : (code & 8 ? -mag[code & 7] : mag[code & 7]);
-                c += (int)qr[32 * g + i] * v;
-            }
-            int dw = 0, m = 1;
-            if (!plainw && Fmt<FMT>::NV) {
-                const uint32_t e4 = srow[16 + 8 * (a.k0 + g / 4) + 2 * (g & 3) + h];
-                dw = nv_dw(e4);
-                m = nv_m(e4);
-            } else if (!plainw) {
-                const uint32_t word = *reinterpret_cast<const uint32_t*>(srow + 8 + 4 * (a.k0 + g / 4));
-                dw = (int)(word & 0xFF);
-                m = (int)((word >> (8 + 6 * (g & 3))) & 63);
-            }
-            const int sh = Fmt<FMT>::W - dw - da;
-            if (sh >= 0) acc += ((int64_t)m * c) << sh;
-        }
-    }
-    return acc;
-}
-
-// y = (i2f(acc) * Sw) * (Sa * 2^-11), then ACC / ASCALE (the reference's epilogue order)
-__device__ __forceinline__ void store_out(const Args& a, int m, int n, int64_t acc, float sw, float sa2) {
-    float y = fmul_f(fmul_f(i2f(acc), sw), sa2);
-    float* o = a.out + (int64_t)m * a.ors + n;
-    if (a.flags & OTPU_ASCALE) y = fadd(fmul(*o, a.alpha[m]), y);
-    else if (a.flags & OTPU_ACC) y = fadd(*o, y);
-    *o = y;
 }
 
 // HI: weights with scale rows (two int8 planes); false: RSC / UNIT weights (w'' = w, one plane)
@@ -427,22 +384,22 @@ __global__ __launch_bounds__(512) void gemm4_kernel(Args a) {
     const int np = __builtin_popcount(dm);
     const int dmin = dm ? __builtin_ctz(dm) : 0, dmax = dm ? 31 - __builtin_clz(dm) : 0;
     // Horner over the planes in int32: |sum_p 2^(dmax - d_p) C_p| <= K 127 128 (2^(dmax - dmin + 1) - 1)
-    const bool fits = dm && (int64_t)a.K * 127 * 128 * ((2ll << (dmax - dmin)) - 1) < (1ll << 31);
+    const bool fits = (int64_t)a.K * 127 * 128 * ((2ll << (dmax - dmin)) - 1) < (1ll << 31);
     const bool single = np == 1 && !over;
-
-    if (dm == 0 || !fits || wide) {
-        // every group drops (acc 0), or the exact VALU path
-        if (streamer) wait_vm<0>();             // (the first walk's first loads, issued before the scan)
-        for (int idx = tid; idx < TM * TN; idx += 512) {
-            const int r = idx / TN, c = idx % TN, m = m0 + r, n = n0 + c;
-            if (m >= a.M || n >= a.N) continue;
-            const int64_t acc = dm ? valu_acc4<FMT>(a, m, n, plainw) : 0;
-            const float sw = unit ? 1.0f : ftz(*reinterpret_cast<const float*>(a.ws + (int64_t)n * a.srs));
-            store_out(a, m, n, acc, sw, sSa2[r]);
-        }
+    if (np < 1 || np > 2 || !fits || wide) {
+        // more activation offsets, or weights past the fold's range: the walk of any offsets, with the
+        // scales applied to the products (prefill_impl.h), on all 8 waves
+        if (streamer) wait_vm<0>();             // (the first loads, issued before the scan)
+        bar();
+        pf::Args pa = {};
+        pa.q = a.q; pa.ldq = a.ldq; pa.Sa = a.Sa; pa.da = a.da; pa.ldda = a.ldda; pa.M = a.M; pa.K = a.K;
+        pa.w = a.w; pa.rs = a.rs; pa.ws = a.ws; pa.srs = a.srs; pa.N = a.N; pa.flags = a.flags;
+        pa.k0 = plainw ? 0 : a.k0;
+        pa.alpha = a.alpha; pa.out = a.out; pa.ors = a.ors; pa.ranges = 1; pa.vec4 = a.vec4;
+        static_assert(pf::Tile<FMT, 2, 2>::LDS <= FT::LDS_BYTES && pf::Tile<FMT, 2, 2>::TM == TM, "the walk's tile");
+        pf::prefill_tile<FMT, 2, 2, false>(pa, lds, m0, n0);
         return;
     }
-
     // The expansion of raw stage s into plane buffer s & 1 for activation plane d.  Every thread
     // of the workgroup expands one of the stage's 512 32-groups, gi = its thread index (row
     // gi / 4, the row's group gi % 4): the multiplying waves do theirs between their MFMAs,
@@ -668,7 +625,7 @@ using namespace otpu;
 int otpu_gemm4_try(const int8_t* q, int64_t ldq, const float* Sa, const uint8_t* da, int64_t ldda, int M, int K,
                    const uint8_t* w, int64_t rs, const uint8_t* ws, int64_t srs, int N, int fmt, int flags, int k0,
                    const float* alpha, float* out, int64_t ors, hipStream_t s) {
-    if ((fmt != OTPU_INT4 && fmt != OTPU_FP4 && fmt != OTPU_NVFP4) || M < 16 || (flags & OTPU_RMAX)) return 1;
+    if ((fmt != OTPU_INT4 && fmt != OTPU_FP4 && fmt != OTPU_NVFP4) || (flags & OTPU_RMAX)) return 1;
     if (fmt == OTPU_NVFP4 && (flags & OTPU_RSC)) return 1;     // (no RSC form: the MM checks refuse it)
     if (((uintptr_t)da & 3) || (ldda % 4) || ((uintptr_t)q & 15) || (ldq % 16) || ((uintptr_t)w & 15) || (rs % 16))
         return 1;

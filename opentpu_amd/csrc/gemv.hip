@@ -175,6 +175,42 @@ int otpu_gemm4_try(const int8_t* q, int64_t ldq, const float* Sa, const uint8_t*
                    const uint8_t* w, int64_t rs, const uint8_t* ws, int64_t srs, int N, int fmt, int flags, int k0,
                    const float* alpha, float* out, int64_t ors, hipStream_t s);
 
+int otpu_batch_try(const int8_t* q, int64_t ldq, const float* Sa, const uint8_t* da, int64_t ldda, int M, int K,
+                   int ranges, const uint8_t* w, int64_t rs, const uint8_t* ws, int64_t srs, int N, int fmt, int flags,
+                   int k0, const float* alpha, float* out, int64_t ors, hipStream_t s);
+
+int otpu_prefill_try(const int8_t* q, int64_t ldq, const float* Sa, const uint8_t* da, int64_t ldda, int M, int K,
+                     int ranges, const uint8_t* w, int64_t rs, const uint8_t* ws, int64_t srs, int N, int fmt, int flags,
+                     int k0, const float* alpha, float* out, int64_t ors, hipStream_t s);
+
+// MM of several activation rows on the MFMA kernels, over `ranges` equal column ranges (their ACC
+// chain): 0 or an error, or > 0 where none of them takes the call (RMAX, offset rows that are not
+// whole words: the GEMV then streams it, a few rows a launch).  act: what is known of the activation
+// offsets (OTPU_ACT_*).  The kernels give the same bits; the lines between them, measured (us):
+//   the batch kernel (no LDS; K split over waves) below 3/4 of a 32 x 128 tile a CU: int8 1024 x 2048
+//     weights at 512 rows 19.2 against the prefill kernel's 19.5, 4096 x 1024 at 128 rows 12.7 / 12.3
+//     (128 tiles), int4 12288 x 2048 at 50 rows 29 / 28 (192 tiles), at 128 rows 48 / 31 (384)
+//   the GEMMs (128 x 128 tiles, one a CU at a time) for plain int8 and 4-bit weights: with one
+//     activation offset they multiply folded operands with no work a product (4096 x 2048 x 8192: rsc
+//     116, int4 214 against the prefill kernel's 161, 308), with several they are the slower (int4
+//     395 / 309).  So they run where the offsets are one (ROW) or unknown, and their last round of
+//     tiles is at least 4/5 full
+//   the prefill kernel for the rest
+static int mm_rows(const int8_t* q, int64_t ldq, const float* Sa, const uint8_t* da, int64_t ldda, int M, int K,
+                   int ranges, const uint8_t* w, int64_t rs, const uint8_t* ws, int64_t srs, int N, int fmt, int flags,
+                   int k0, int act, const float* alpha, float* out, int64_t ors, hipStream_t s) {
+    const int64_t n128 = (N + 127) / 128, tiles = (M + 127) / 128 * n128, cus = otpu_cu_count();
+    if ((M + 31) / 32 * n128 < cus * 3 / 4)
+        return otpu_batch_try(q, ldq, Sa, da, ldda, M, K, ranges, w, rs, ws, srs, N, fmt, flags, k0, alpha, out, ors, s);
+    if (ranges == 1 && act != OTPU_ACT_MX && tiles * 5 / 4 >= (tiles + cus - 1) / cus * cus) {
+        int rc = otpu_gemm_try(q, ldq, Sa, da, ldda, M, K, w, rs, ws, srs, N, fmt, flags, k0, alpha, out, ors, s);
+        if (rc <= 0) return rc;
+        rc = otpu_gemm4_try(q, ldq, Sa, da, ldda, M, K, w, rs, ws, srs, N, fmt, flags, k0, alpha, out, ors, s);
+        if (rc <= 0) return rc;
+    }
+    return otpu_prefill_try(q, ldq, Sa, da, ldda, M, K, ranges, w, rs, ws, srs, N, fmt, flags, k0, alpha, out, ors, s);
+}
+
 extern "C" int otpu_mm(const int8_t* q, int64_t ldq, const float* Sa, const uint8_t* da, int64_t ldda,
                        int M, int K, const uint8_t* w, int64_t rs, const uint8_t* ws, int64_t srs, int N,
                        int fmt, int flags, int k0, const float* alpha, float* out, int64_t ors,
@@ -186,12 +222,9 @@ extern "C" int otpu_mm(const int8_t* q, int64_t ldq, const float* Sa, const uint
     if ((flags & OTPU_RMAX) && !rowmax) return otpu_fail(OTPU_EINVAL, "mm: RMAX without rowmax");
     hipStream_t s = (hipStream_t)stream;
     if (M > 4) {
-        rc = otpu_gemm_try(q, ldq, Sa, da, ldda, M, K, w, rs, ws, srs, N, fmt, flags & ~OTPU_PAIR, k0, alpha,
-                           out, ors, s);
-        if (rc <= 0) return rc;                       // handled (or failed); > 0: not this path
-        rc = otpu_gemm4_try(q, ldq, Sa, da, ldda, M, K, w, rs, ws, srs, N, fmt, flags & ~OTPU_PAIR, k0, alpha,
-                            out, ors, s);
-        if (rc <= 0) return rc;
+        rc = mm_rows(q, ldq, Sa, da, ldda, M, K, 1, w, rs, ws, srs, N, fmt, flags & ~OTPU_PAIR, k0, OTPU_ACT_ANY, alpha,
+                     out, ors, s);
+        if (rc <= 0) return rc;                       // handled (or failed); > 0: not these paths
     }
     MMArgs a = make_args(q, ldq, Sa, da, ldda, M, K, w, rs, ws, srs, N, flags, k0);
     a.alpha = alpha; a.out = out; a.ors = ors;
@@ -261,6 +294,11 @@ extern "C" int otpu_mm_ranges(const int8_t* q, int64_t ldq, const float* Sa, con
     if (!Sa || !part || !out || ors < N) return otpu_fail(OTPU_EINVAL, "mm_ranges: Sa / part / out NULL or ors < N");
     if (!al(part, 4)) return otpu_fail(OTPU_EALIGN, "mm_ranges: part");
     hipStream_t s = (hipStream_t)stream;
+    if (M > 4) {
+        rc = mm_rows(q, ldq, Sa, da, ldda, M, K, R, w, rs, ws, srs, N, fmt, flags & ~OTPU_PAIR, k0, OTPU_ACT_ANY, nullptr,
+                     out, ors, s);
+        if (rc <= 0) return rc;
+    }
     MMArgs a = make_args(q, ldq, Sa, da, ldda, M, width, w, rs, ws, srs, N, flags & ~OTPU_ACC, k0);
     a.out = part; a.ors = N;
     a.q_bs = width; a.sa_bs = M; a.da_bs = width / 32;
@@ -272,6 +310,30 @@ extern "C" int otpu_mm_ranges(const int8_t* q, int64_t ldq, const float* Sa, con
     sum_parts<<<(unsigned)((tot + 255) / 256), 256, 0, s>>>(part, (int64_t)M * N, R, M, N, (flags & OTPU_ACC) != 0,
                                                             out, ors);
     return otpu_launch_check("mm_ranges");
+}
+
+extern "C" int otpu_mm_dot(const int8_t* q, int64_t ldq, const float* Sa, const uint8_t* da, int64_t ldda, int M, int K,
+                           int width, const uint8_t* w, int64_t rs, const uint8_t* ws, int64_t srs, int N, int fmt,
+                           int flags, int k0, int act, const float* alpha, float* out, int64_t ors,
+                           otpu_stream_t stream) {
+    const int chunk = fmt == OTPU_INT8 ? OTPU_D : 2 * OTPU_D;
+    if (width < 1 || K % width || (width < K && (width < chunk || width % chunk)))
+        return otpu_fail(OTPU_EINVAL, "mm_dot: ranges of %d over K %d (multiples of %d for this format)", width, K, chunk);
+    if (flags & OTPU_RMAX) return otpu_fail(OTPU_EINVAL, "mm_dot: no RMAX");
+    if (act < OTPU_ACT_ANY || act > OTPU_ACT_MX) return otpu_fail(OTPU_EINVAL, "mm_dot: act %d", act);
+    int rc = check_mm("mm_dot", q, ldq, da, ldda, M, K, w, rs, ws, srs, N, fmt, flags, k0);
+    if (rc) return rc;
+    if (!Sa || !out || ors < N) return otpu_fail(OTPU_EINVAL, "mm_dot: Sa / out NULL or ors < N");
+    if ((flags & OTPU_ASCALE) && !alpha) return otpu_fail(OTPU_EINVAL, "mm_dot: ASCALE without alpha");
+    hipStream_t s = (hipStream_t)stream;
+    const int R = K / width;
+    if (R == 1 && M <= 4) {
+        MMArgs a = make_args(q, ldq, Sa, da, ldda, M, K, w, rs, ws, srs, N, flags, k0);
+        a.alpha = alpha; a.out = out; a.ors = ors;
+        return launch_gemv(a, fmt, 1, s);
+    }
+    rc = mm_rows(q, ldq, Sa, da, ldda, M, K, R, w, rs, ws, srs, N, fmt, flags & ~OTPU_PAIR, k0, act, alpha, out, ors, s);
+    return rc > 0 ? otpu_fail(OTPU_EALIGN, "mm_dot: offset rows of whole words (da, ldda multiples of 4)") : rc;
 }
 
 namespace otpu {

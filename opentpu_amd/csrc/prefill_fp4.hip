@@ -1,0 +1,8 @@
+// The prefill MM's kernels for fp4 weights.
+#include "prefill_impl.h"
+
+namespace otpu {
+namespace pf {
+template void launch_fmt<OTPU_FP4>(const Args& a, int ms, hipStream_t s);
+}  // namespace pf
+}  // namespace otpu

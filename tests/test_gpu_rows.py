@@ -1,0 +1,163 @@
+"""MM of several activation rows on the MFMA kernels -- the batch kernel (csrc/batch_impl.h), the
+prefill kernel (csrc/prefill_impl.h) and the GEMMs with the prefill walk inside them -- and
+otpu_mm_dot's ranges, against the C oracle bit for bit (`opentpu/isasim.py:749-910`,
+`opentpu/compiler.py:2686-2720`).  Sizes at the edges of tiles, of the K splits and of the rules
+that pick a kernel; offsets inside and outside the kernels' int32 windows."""
+import numpy as np
+import pytest
+
+from conftest import same_bits
+from oracle import cpu as OC
+from oracle import fp32 as F
+from oracle import mm as MM
+from test_gpu_gemm4 import activations, say, weights
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.fixture(scope="module")
+def X():
+    import torch
+    assert torch.cuda.is_available(), "GPU tests need a GPU"
+    from opentpu_amd import _lib
+    _lib.load()
+    return _lib
+
+
+def mm_dot(X, q, Sa, da, rows, srows, fmt, K, width, flags=0, k0=0, act=0, old=None, alpha=None, N=None):
+    M, N = q.shape[0], rows.shape[0] if N is None else N
+    qd, Sd, dd = X.dev(q, np.int8), X.dev(Sa, np.float32), X.dev(da, np.uint8)
+    w, ws = X.dev(rows, np.uint8), X.dev(srows, np.uint8)
+    al = X.dev(alpha, np.float32) if alpha is not None else None
+    out = X.empty((M, N), np.float32) if old is None else X.dev(old, np.float32).clone()
+    X.call("otpu_mm_dot", X.ptr(qd), K, X.ptr(Sd), X.ptr(dd), K // 32, M, K, width, X.ptr(w), w.shape[1], X.ptr(ws),
+           ws.shape[1], N, X.FMT[fmt], flags, k0, act, X.ptr(al), X.ptr(out), N, X.stream())
+    return X.host(out)
+
+
+def int8_weights(rng, N, K, wk):
+    from oracle import formats as Q
+    W = rng.standard_normal((N, K)).astype(np.float32) * 0.02
+    if wk == "spread":                                    # block offsets over several octaves
+        W *= np.exp2(-rng.integers(0, 7, (N, K // 128))).repeat(128, 1).astype(np.float32)
+    if wk == "far":                                       # ... past every window
+        W *= np.exp2(-rng.integers(0, 20, (N, K // 128))).repeat(128, 1).astype(np.float32)
+    return Q.pack_rsc(W) if wk == "rsc" else Q.pack_int8x(W)
+
+
+def operands(rng, M, N, K, fmt, wk, ak, k0=0):
+    q, Sa, da = activations(rng, M, K, ak)
+    if fmt == "int8":
+        rows, srows = int8_weights(rng, N, K + 128 * k0, wk)
+        rows = np.ascontiguousarray(rows[:, 128 * k0:])
+    else:
+        rows, srows = weights(rng, N, K, fmt, wk, k0)
+    return q, Sa, da, rows, srows, {"rsc": MM.RSC, "unit": MM.UNIT}.get(wk, 0)
+
+
+WIN = (0, 3, 6, 8)                                        # offsets up to and past the block windows
+KINDS = [("int8", "x8", "mx"), ("int8", "spread", "mx"), ("int8", "far", WIN), ("int8", "rsc", (0, 20)),
+         ("int4", "x4", "mx"), ("int4", "spread", WIN), ("int4", "rsc", "mx"), ("fp4", "wide", "mx"),
+         ("fp4", "x4", (2, 5, 9)), ("nvfp4", "x4", "mx"), ("nvfp4", "tiny", WIN), ("nvfp4", "unit", "mx"),
+         ("nvfp4", "wider", "wide")]
+
+
+@pytest.mark.parametrize("M,N,K", [(5, 1, 128), (16, 100, 1024), (17, 257, 384), (33, 1000, 2048), (50, 2500, 256)])
+@pytest.mark.parametrize("fmt,wk,ak", KINDS)
+def test_batch(X, M, N, K, fmt, wk, ak):
+    from opentpu_amd import mxu
+    rng = np.random.default_rng(M + N + K)
+    q, Sa, da, rows, srows, fl = operands(rng, M, N, K, fmt, wk, ak)
+    say("batch", M, N, K, fmt, wk, ak)
+    got = mxu.mm(q, Sa, da, rows, srows, fmt, K, rsc=wk == "rsc", unit=wk == "unit")
+    assert same_bits(got, OC.mm(q, Sa, da, rows, srows, fmt, K, flags=fl))
+
+
+@pytest.mark.parametrize("M,N,K,act", [(100, 8100, 256, 2), (500, 8100, 384, 2), (500, 8100, 384, 0), (129, 26000, 128, 1)])
+@pytest.mark.parametrize("fmt,wk,ak", KINDS + [("int8", "rsc", "mx"), ("int8", "rsc", WIN), ("int8", "x8", "row"),
+                                               ("fp4", "x4", "row"), ("nvfp4", "x4", "row")])
+def test_prefill(X, M, N, K, act, fmt, wk, ak):
+    """act 2: the prefill kernel (32 and 64 rows a tile); 0 and 1: the GEMMs, ragged last tiles."""
+    rng = np.random.default_rng(M + N + K)
+    q, Sa, da, rows, srows, fl = operands(rng, M, N, K, fmt, wk, ak)
+    say("prefill", M, N, K, act, fmt, wk, ak)
+    got = mm_dot(X, q, Sa, da, rows, srows, fmt, K, K, fl, act=act)
+    assert same_bits(got, OC.mm(q, Sa, da, rows, srows, fmt, K, flags=fl))
+
+
+@pytest.mark.parametrize("fmt", ["int8", "int4", "nvfp4"])
+def test_prefill_long_sums(X, fmt):
+    """Sums that leave int32 inside the walk: every product at its largest over K = 16384."""
+    rng = np.random.default_rng(3)
+    M, N, K = 512, 8192, 16384
+    _, _, _, rows, srows, _ = operands(rng, 1, N, 256, fmt, "x8" if fmt == "int8" else "x4", "mx")
+    rep = K // 256
+    rows = np.tile(rows, (1, rep))
+    rows[:] = {"int8": 0x7F, "int4": 0x77, "nvfp4": 0x77}[fmt]
+    KB = K // 128
+    if fmt == "int8":
+        srows = np.concatenate([srows[:, :4], np.zeros((N, KB), np.uint8)], 1)
+    elif fmt == "int4":
+        word = np.full((N, KB), sum(63 << (8 + 6 * b) for b in range(4)), np.uint32)
+        srows = np.concatenate([srows[:, :4], np.zeros((N, 4), np.uint8), word.view(np.uint8).reshape(N, 4 * KB)], 1)
+    else:
+        srows = np.concatenate([srows[:, :16], np.full((N, 8 * KB), 0x7F, np.uint8)], 1)
+    q = np.full((M, K), 127, np.int8)
+    q[1::2] = -127
+    da = rng.integers(0, 3, (M, K // 32)).astype(np.uint8)
+    Sa = np.ones(M, np.float32)
+    say("prefill long", fmt)
+    got = mm_dot(X, q, Sa, da, rows, srows, fmt, K, K, act=2)
+    rows_s, srows_s = np.ascontiguousarray(rows[:40]), np.ascontiguousarray(srows[:40])
+    assert same_bits(got[:, :40], OC.mm(q, Sa, da, rows_s, srows_s, fmt, K))
+
+
+@pytest.mark.parametrize("M,N", [(1, 300), (4, 70), (5, 1024), (40, 999), (200, 12000), (257, 17000)])
+@pytest.mark.parametrize("fmt,K,width", [("int8", 1152, 384), ("int8", 1536, 128), ("int4", 768, 256), ("fp4", 3072, 256),
+                                         ("nvfp4", 1536, 768)])
+def test_dot_ranges(X, M, N, fmt, K, width):
+    """A QACT range per MM, the MMs' outputs added in range order; ACC's old values first."""
+    rng = np.random.default_rng(M + N + K)
+    if M * N * K > 2e9:
+        N = int(2e9 / M / K) // 8 * 8 + 3
+    R = K // width
+    _, _, _, rows, srows, _ = operands(rng, 1, N, K, fmt, "spread", "mx")
+    x = (rng.standard_normal((M, K)) * rng.standard_normal((M, K))).astype(np.float32)
+    parts = [F.quantize_mx(x[:, r * width:(r + 1) * width], 32) for r in range(R)]
+    q, da = np.concatenate([p[0] for p in parts], 1), np.concatenate([p[2] for p in parts], 1)
+    Sa = np.stack([p[1] for p in parts])
+    old = rng.standard_normal((M, N)).astype(np.float32)
+    say("dot ranges", M, N, fmt, K, width)
+    bpb = 128 if fmt == "int8" else 64
+    for flags, want in ((0, None), (MM.ACC, old)):
+        got = mm_dot(X, q, Sa, da, rows, srows, fmt, K, width, flags, act=2, old=None if want is None else old)
+        for r in range(R):
+            kb = r * width // 128
+            rw = np.ascontiguousarray(rows[:, kb * bpb:(kb + width // 128) * bpb])
+            f = 0 if want is None else MM.ACC
+            want = OC.mm(np.ascontiguousarray(parts[r][0]), parts[r][1], parts[r][2], rw, srows, fmt, width, flags=f, k0=kb, old=want)
+        assert same_bits(got, want)
+
+
+@pytest.mark.parametrize("M,N", [(20, 200), (200, 12000)])
+def test_rows_acc_ascale_k0(X, M, N):
+    from opentpu_amd import mxu
+    rng = np.random.default_rng(M)
+    K = 256
+    q, Sa, da, rows, srows, _ = operands(rng, M, N, K, "fp4", "x4", "mx", k0=2)
+    old = rng.standard_normal((M, N)).astype(np.float32)
+    alpha = rng.standard_normal(M).astype(np.float32)
+    say("rows acc / ascale / k0", M, N)
+    got = mxu.mm(q, Sa, da, rows, srows, "fp4", K, k0=2, acc=old)
+    assert same_bits(got, OC.mm(q, Sa, da, rows, srows, "fp4", K, flags=MM.ACC, k0=2, old=old))
+    zs = np.zeros((N, 8), np.uint8)
+    got = mm_dot(X, q, Sa, da, rows, zs, "fp4", K, K, MM.UNIT | MM.ACC | MM.ASCALE, act=2, old=old, alpha=alpha)
+    assert same_bits(got, OC.mm(q, Sa, da, rows, zs, "fp4", K, flags=MM.UNIT | MM.ACC | MM.ASCALE, old=old, alpha=alpha))
+
+
+def test_mm_dot_refuses(X):
+    rng = np.random.default_rng(1)
+    q, Sa, da, rows, srows, _ = operands(rng, 6, 32, 512, "int4", "x4", "mx")
+    for kw in ({"width": 128}, {"width": 300}, {"width": 512, "act": 3}, {"width": 512, "flags": MM.RMAX}):
+        with pytest.raises(X.OtpuError):
+            mm_dot(X, q, Sa, da, rows, srows, "int4", 512, kw["width"], kw.get("flags", 0), act=kw.get("act", 0))
