@@ -157,17 +157,20 @@ def quantize_ranges(x, ranges=None, row_mode: bool = False):
     ranges = [K] if ranges is None else list(ranges)
     if sum(ranges) != K or any(r % D for r in ranges):
         raise ValueError(f"quantize_ranges: ranges {ranges} over {K} columns")
-    T = X.torch()
     q = X.empty((M, K), np.int8)
     da = X.empty((M, K // 32), np.uint8)
     Sa = X.empty((len(ranges), M), np.float32)
+    flags = X.Q_ROW if row_mode else 0
+    if len(ranges) > 1 and min(ranges) == max(ranges):    # equal ranges: one launch
+        X.call("otpu_qact_ranges", X.ptr(xd), None, M, K, K, ranges[0], 32, flags, None, None, X.ptr(q), K, X.ptr(Sa),
+               X.ptr(da), K // 32, X.stream())
+        return q, Sa, da, ranges
     c0 = 0
     for i, w in enumerate(ranges):
         xs = xd[:, c0:c0 + w]
-        X.call("otpu_qact", X.ptr(xs), M, w, K, 32, X.Q_ROW if row_mode else 0, None, None, C_ptr(q, c0), K,
+        X.call("otpu_qact", X.ptr(xs), M, w, K, 32, flags, None, None, C_ptr(q, c0), K,
                X.ptr(Sa[i]), C_ptr(da, c0 // 32), K // 32, None, 0, X.stream())
         c0 += w
-    del T
     return q, Sa, da, ranges
 
 
@@ -176,29 +179,82 @@ def C_ptr(t, off: int):
     return ctypes.c_void_p(t.data_ptr() + off * t.element_size())
 
 
+# one activation row quantized inside the GEMV (otpu_mm_qin) instead of by a launch of its own: every
+# workgroup quantizes the row again, which pays while the weights are few (4096 x 1024 int4: one launch
+# of 4.7 us for two of 2.9 and 3.0; the LM head's 262144 rows: 160 us for 3 + 107)
+QIN_ROWS = 16384
+QIN_COLS = 16384                                          # columns otpu_mm_qin's prologue holds
+FOLD_COLS = 8192                                          # ... and otpu_mm_qin_fold's
+
+
+def _dot_row(x, w: QWeight, ranges, out) -> bool:
+    """One fp32 row x (a contiguous device tensor [1, K]) @ w^T into out in one launch, QACT and the
+    ranges' ACC chain inside; False where no such kernel takes the call."""
+    K, chunk = w.K, (D if w.fmt == "int8" else 2 * D)
+    if w.N > QIN_ROWS or x.data_ptr() % 16 or K % chunk:
+        return False
+    ws, srs = (0, 0) if w.srows is None else (w.srows.data_ptr(), w.srows.shape[1])
+    fl = _flags(w.srows is None, w.rsc)
+    if len(ranges) == 1:
+        if K > QIN_COLS:
+            return False
+        X.call("otpu_mm_qin", x.data_ptr(), None, None, None, 1, 0, K, K, w.rows.data_ptr(), w.rows.shape[1], ws, srs,
+               w.N, X.FMT[w.fmt], fl, 0, out.data_ptr(), w.N, 0, X.stream())
+        return True
+    width = ranges[0]
+    if fl or w.fmt == "int8" or K > FOLD_COLS or min(ranges) != max(ranges) or width % chunk:
+        return False
+    X.call("otpu_mm_qin_fold", x.data_ptr(), None, None, None, K, width, w.rows.data_ptr(), w.rows.shape[1], ws, srs,
+           w.N, X.FMT[w.fmt], 0, 0, out.data_ptr(), X.stream())
+    return True
+
+
 def dot(x, w: QWeight, acc=None, out=None, ranges=None, row_mode: bool = False, rowmax: bool = False,
         acc_scale=None):
     """x [M, K] (fp32, quantized here, or a (q, Sa, da, ranges) operand from quantize_ranges)
     @ w^T -> [M, N] fp32, as `ol.dot` lowers it: one QACT per range, one MM per range, the
     first overwriting (or ACC into `acc`, or ASCALE with acc_scale), the rest ACC.  The
     4-bit formats need ranges that start on even blocks (a 128-byte chunk holds two blocks).
-    rowmax: also return the row maxima of the final sums (MM RMAX on the last range)."""
+    rowmax: also return the row maxima of the final sums (MM RMAX on the last range).
+
+    Equal ranges run as one QACT launch and one MM launch (otpu_mm_dot: the ACC chain inside), one
+    fp32 row as a single launch where a kernel does both; anything else as a launch per range."""
     numpy_in = X.is_numpy(x)
-    if isinstance(x, tuple):
-        q, Sa, da, ranges = x
-    else:
-        q, Sa, da, ranges = quantize_ranges(x, ranges, row_mode)
-    M, K = q.shape
-    if K != w.K:
-        raise ValueError(f"dot: K mismatch {K} vs {w.K}")
     if acc is not None and out is not None:
         raise ValueError("dot: give either acc= or out=")
     N = w.N
+    operand = isinstance(x, tuple)
+    xd = None
+    if not operand:
+        xd = X.dev(x, np.float32)
+        K = xd.shape[1]
+        if K != w.K:
+            raise ValueError(f"dot: K mismatch {K} vs {w.K}")
+        if xd.shape[0] == 1 and not (row_mode or rowmax) and acc is None and acc_scale is None:
+            rl = [K] if ranges is None else list(ranges)
+            if sum(rl) == K and not any(r % D for r in rl):
+                y = out if out is not None else X.empty((1, N), np.float32)
+                if _dot_row(xd, w, rl, y):
+                    return X.host(y) if numpy_in else y
+        q, Sa, da, ranges = quantize_ranges(xd, ranges, row_mode)
+    else:
+        q, Sa, da, ranges = x
+    M, K = q.shape
+    if K != w.K:
+        raise ValueError(f"dot: K mismatch {K} vs {w.K}")
     y = X.dev(acc, np.float32) if acc is not None else (out if out is not None else X.empty((M, N), np.float32))
     unit = w.srows is None
+    al = X.dev(acc_scale, np.float32) if acc_scale is not None else None
+    chunk = D if w.fmt == "int8" else 2 * D
+    width = ranges[0]
+    if not rowmax and (len(ranges) == 1 or (min(ranges) == max(ranges) and width % chunk == 0)):
+        act = X.ACT_ANY if operand else (X.ACT_ROW if row_mode else X.ACT_MX)
+        X.call("otpu_mm_dot", q.data_ptr(), K, Sa.data_ptr(), da.data_ptr(), K // 32, M, K, width, w.rows.data_ptr(),
+               w.rows.shape[1], 0 if unit else w.srows.data_ptr(), 0 if unit else w.srows.shape[1], N, X.FMT[w.fmt],
+               _flags(unit, w.rsc, acc is not None, al is not None), 0, act, X.ptr(al), y.data_ptr(), N, X.stream())
+        return X.host(y) if numpy_in else y
     bpb = D if w.fmt == "int8" else D // 2
     rm = X.empty((M,), np.float32) if rowmax else None
-    al = X.dev(acc_scale, np.float32) if acc_scale is not None else None
     c0 = 0
     for i, width in enumerate(ranges):
         k0 = c0 // D
