@@ -38,8 +38,108 @@ __device__ __forceinline__ int e2m1_code(double v) {
     return (a > 0.25) + (a >= 0.75) + (a > 1.25) + (a >= 1.75) + (a > 2.5) + (a >= 3.5) + (a > 5.0);
 }
 
+// The candidates' errors without a division.  Every candidate is a float64 division, a rounding
+// and a squared error an element, and those divisions were nearly all of the packers' time (int4
+// 6144 x 2048: 156 us, where a copy of its bytes takes 11).  Here an element's quotient is its
+// product with the scale's reciprocal, off by less than 2^-50 of itself, so
+//   - the rounding goes another way only within 2^-50 |x / s| of a midpoint, where the squared
+//     error of either side is the same within 2^-48 |x| s (half a step is 1 at most);
+//   - e = g s - |x| is off by 2^-52 |x|, its square by 2^-51 |e| |x| + 2^-104 x^2;
+// and a sum over n <= 32 elements, with its own roundings, by less than 2^-45 (E + X + 32 s^2), X
+// the sum of x^2 (by Cauchy: sum |x| s <= (X + n s^2) / 2).  A winner ahead of every other
+// candidate by 2^-40 of both bounds together, s the largest tried, is the exact search's;
+// anything closer (equal errors among it) is searched in the reference's arithmetic, and so are
+// infinities and NaN.  Measured, 6144 x 2048: int4 156 -> 42 us, fp4 320 -> 71, nvfp4 285 -> 90; one
+// row of 2048: 31 -> 10, 75 -> 15, 64 -> 23; weights on half-steps, whose candidates tie in every
+// wave: 157 -> 44, 322 -> 73, 286 -> 92.  Still bound by arithmetic: 5 to 8 float64 operations an
+// element and candidate.
+constexpr double SEARCH_TOL = 0x1p-40;
+
+// the grid value nearest to a >= 0 (a midpoint to either side); *half: half the step there.  E2M1:
+// steps of 1/2 below 2, then 1 and 2, by adding and subtracting 1.5 2^52 steps
 template <bool E2M1>
-__global__ __launch_bounds__(64) void pack_x4_kernel(const float* __restrict__ W, int K, int64_t ldw,
+__device__ __forceinline__ double near_grid(double a, double* half) {
+    if (!E2M1) {
+        *half = 0.5;
+        return fmin(__builtin_rint(a), 7.0);
+    }
+    const int e = max(__double2hiint(a) & 0x7ff00000, 0x3ff00000);               // a's binade, 1 at least
+    const double c = __hiloint2double(e + (0x43280000 - 0x3ff00000), 0);
+    *half = __hiloint2double(e - 0x00200000, 0);
+    return fmin((a + c) - c, 6.0);
+}
+
+template <bool E2M1, int NE>
+__device__ __forceinline__ double near_error(const double (&xv)[NE], double s) {
+    const double r = 1.0 / s;
+    double p[4] = {0.0, 0.0, 0.0, 0.0};
+#pragma unroll
+    for (int i = 0; i < NE; ++i) {
+        double h;
+        const double g = near_grid<E2M1>(fabs(xv[i]) * r, &h), e = __builtin_fma(-g, s, fabs(xv[i]));
+        p[i & 3] = __builtin_fma(e, e, p[i & 3]);
+    }
+    return (p[0] + p[1]) + (p[2] + p[3]);
+}
+
+template <int NE>
+__device__ __forceinline__ double sum_squares(const double (&xv)[NE]) {
+    double X = 0.0;
+#pragma unroll
+    for (int i = 0; i < NE; ++i) X = __builtin_fma(xv[i], xv[i], X);
+    return X;
+}
+
+// the codes of xv / s from the same products; false if a quotient is within 2^-40 of a midpoint
+// (the reference's (grid(x / s) s) / s is within 2^-52 of the grid value, and has its code)
+template <bool E2M1, int NE>
+__device__ __forceinline__ bool near_codes(const double (&xv)[NE], double s, uint32_t (&word)[NE / 8]) {
+    const double r = 1.0 / s;
+    bool clear = true;
+#pragma unroll
+    for (int w = 0; w < NE / 8; ++w) word[w] = 0;
+#pragma unroll
+    for (int i = 0; i < NE; ++i) {
+        double h;
+        const double a = fabs(xv[i]) * r, g = near_grid<E2M1>(a, &h);
+        clear &= fabs(fabs(a - g) - h) >= 0x1p-40;        // (past the last grid value: never taken for one)
+        uint32_t code;
+        if (!E2M1) {
+            const int k = (int)g;
+            code = (uint32_t)(xv[i] < 0.0 ? -k : k) & 15;
+        } else {
+            const int k = (int)(2.0 * g), mag = k <= 4 ? k : (k == 6 ? 5 : (k == 8 ? 6 : 7));
+            code = (uint32_t)(mag | (xv[i] < 0.0 && mag != 0 ? 8 : 0));
+        }
+        word[i >> 3] |= code << (4 * (i & 7));
+    }
+    return clear;
+}
+
+// one of a row's sub-blocks (past the row: zeros); its float64 magnitude
+template <int NE>
+__device__ __forceinline__ double load_block(const float* x, bool ok, double (&xv)[NE]) {
+    float v[NE];
+    if (ok && ((uintptr_t)x & 15) == 0) {
+#pragma unroll
+        for (int i = 0; i < NE / 4; ++i) *reinterpret_cast<float4*>(v + 4 * i) = *reinterpret_cast<const float4*>(x + 4 * i);
+    } else {
+#pragma unroll
+        for (int i = 0; i < NE; ++i) v[i] = ok ? x[i] : 0.0f;
+    }
+    float m = 0.0f;
+#pragma unroll
+    for (int i = 0; i < NE; ++i) {
+        m = fmaxf(m, fabsf(v[i]));
+        xv[i] = (double)v[i];
+    }
+    return (double)m;
+}
+
+// three waves a SIMD: the 32 float64 elements a lane holds take 64 registers, the search's eight or
+// so in flight the rest
+template <bool E2M1>
+__global__ __launch_bounds__(64, 3) void pack_x4_kernel(const float* __restrict__ W, int K, int64_t ldw,
                                                      uint8_t* __restrict__ rows, int64_t rs,
                                                      uint8_t* __restrict__ srows, int64_t srs, Search sr) {
     const int row = blockIdx.x, lane = threadIdx.x;
@@ -47,11 +147,10 @@ __global__ __launch_bounds__(64) void pack_x4_kernel(const float* __restrict__ W
     const int NS = K / 32, KB = K / 128;
     const double qmax = E2M1 ? 6.0 : 7.0;
 
-    double top = 0.0;
-    for (int s = lane; s < NS; s += 64) {
-        double m = 0.0;
-        for (int i = 0; i < 32; ++i) m = fmax(m, fabs((double)x[32 * s + i]));
-        top = fmax(top, m / qmax);
+    double xv[32], top = 0.0, amax = 0.0;
+    for (int s = lane; s < (NS + 63) / 64 * 64; s += 64) {
+        amax = load_block(x + 32 * s, s < NS, xv);
+        top = fmax(top, amax / qmax);
     }
     for (int o = 32; o > 0; o >>= 1) top = fmax(top, __shfl_xor(top, o, 64));
     const double Sw = top == 0.0 ? 1.0 : (double)(float)(top / 63.0);
@@ -61,13 +160,7 @@ __global__ __launch_bounds__(64) void pack_x4_kernel(const float* __restrict__ W
     for (int s0 = 0; s0 < NS; s0 += 64) {               // uniform: every lane shuffles
         const int s = s0 + lane;
         const bool ok = s < NS;
-        double xv[32];
-        double amax = 0.0;
-#pragma unroll
-        for (int i = 0; i < 32; ++i) {
-            xv[i] = ok ? (double)x[32 * s + i] : 0.0;
-            amax = fmax(amax, fabs(xv[i]));
-        }
+        if (NS > 64) amax = load_block(x + 32 * s, ok, xv);           // (else still held)
         const double sb = amax / qmax;
         double bmax = fmax(sb, __shfl_xor(sb, 1, 64));
         bmax = fmax(bmax, __shfl_xor(bmax, 2, 64));
@@ -84,36 +177,71 @@ __global__ __launch_bounds__(64) void pack_x4_kernel(const float* __restrict__ W
         }
         const double unit = Sw * exp2(-d);
         const double m0 = sb / unit;
-        double best_m = 0.0, best_e = 0.0;
+        auto mult = [&](int c) {
+            const double m = __builtin_rint(m0 * sr.f[c]);
+            return m < 1.0 ? 1.0 : (m > 63.0 ? 63.0 : m);
+        };
+        auto at = [&](int i) { return ok ? (double)x[32 * s + i] : 0.0; };    // read again: seldom used
+        const double X = sum_squares(xv), inf = __builtin_inf();
+        double best_m = 0.0, best_e = inf, next_e = inf, last = 0.0;
+#pragma unroll 1
         for (int c = 0; c < 13; ++c) {
-            double m = __builtin_rint(m0 * sr.f[c]);
-            m = m < 1.0 ? 1.0 : (m > 63.0 ? 63.0 : m);
-            const double sc = unit * m;
-            double p[8];
+            const double m = mult(c);
+            if (m == last) continue;                     // (multipliers never fall: an equal one is the last)
+            last = m;
+            const double E = near_error<E2M1>(xv, unit * m);
+            if (E < best_e) { next_e = best_e; best_e = E; best_m = m; }
+            else next_e = fmin(next_e, E);
+        }
+        // the largest scale tried bounds the errors' errors; unit 0, infinities and NaN are not plain
+        const double s1 = unit * last, reach = best_e + SEARCH_TOL * (best_e + X + 64.0 * (s1 * s1));
+        const bool plain = m0 < 1e6 && X < inf;
+        if (!(plain && next_e > reach)) {
+            bool first = true;
+            last = 0.0;
+#pragma unroll 1
+            for (int c = 0; c < 13; ++c) {
+                const double m = mult(c);
+                if (m == last) continue;
+                last = m;
+                const double sc = unit * m;
+                if (plain && near_error<E2M1>(xv, sc) > reach) continue;
+                double p[8] = {0.0, 0.0, 0.0, 0.0, 0.0, 0.0, 0.0, 0.0};      // (0 + e is e)
+#pragma unroll 1
+                for (int i0 = 0; i0 < 32; i0 += 8) {
 #pragma unroll
-            for (int i = 0; i < 32; ++i) {
-                const double q = grid_value(xv[i] / sc, E2M1) * sc;
-                const double e = (q - xv[i]) * (q - xv[i]);
-                if (i < 8) p[i] = e;
-                else p[i & 7] = p[i & 7] + e;
+                    for (int i = 0; i < 8; ++i) {
+                        const double v = at(i0 + i), q = grid_value(v / sc, E2M1) * sc;
+                        p[i] = p[i] + (q - v) * (q - v);
+                    }
+                }
+                const double err = ((p[0] + p[1]) + (p[2] + p[3])) + ((p[4] + p[5]) + (p[6] + p[7]));
+                if (first || err < best_e) { best_e = err; best_m = m; }
+                first = false;
             }
-            const double err = ((p[0] + p[1]) + (p[2] + p[3])) + ((p[4] + p[5]) + (p[6] + p[7]));
-            if (c == 0 || err < best_e) { best_e = err; best_m = m; }
         }
         // element codes of the winner: g = (grid(x/s) * s) / (unit * m)
         const double sc = unit * best_m;
-        uint32_t word[4] = {0, 0, 0, 0};
+        uint32_t word[4];
+        if (!(near_codes<E2M1>(xv, sc, word) && plain)) {
+#pragma unroll 1
+            for (int w = 0; w < 4; ++w) {
+                uint32_t u = 0;
 #pragma unroll
-        for (int i = 0; i < 32; ++i) {
-            const double g = (grid_value(xv[i] / sc, E2M1) * sc) / sc;
-            uint32_t code;
-            if (!E2M1) {
-                code = (uint32_t)((long long)__builtin_rint(g) & 15);
-            } else {
-                const int mag = e2m1_code(g);
-                code = (uint32_t)(mag | ((signbit(g) && mag != 0) ? 8 : 0));
+                for (int i = 0; i < 8; ++i) {
+                    const double g = (grid_value(at(8 * w + i) / sc, E2M1) * sc) / sc;
+                    uint32_t code;
+                    if (!E2M1) {
+                        code = (uint32_t)((long long)__builtin_rint(g) & 15);
+                    } else {
+                        const int mag = e2m1_code(g);
+                        code = (uint32_t)(mag | ((signbit(g) && mag != 0) ? 8 : 0));
+                    }
+                    u |= code << (4 * i);
+                }
+#pragma unroll
+                for (int k = 0; k < 4; ++k) word[k] = k == w ? u : word[k];
             }
-            word[i >> 3] |= code << (4 * (i & 7));
         }
         if (ok) *reinterpret_cast<uint4*>(erow + 16 * s) = make_uint4(word[0], word[1], word[2], word[3]);
         // the block's scale word: dw | m_b << (8 + 6 b), assembled by the block's first lane
@@ -176,45 +304,78 @@ __global__ __launch_bounds__(64) void pack_nv_kernel(const float* __restrict__ W
     for (int o = 32; o > 0; o >>= 1) am = fmaxf(am, __shfl_xor(am, o, 64));
     double ts = (double)am / 2688.0;
     ts = (double)(float)(ts == 0.0 ? 1.0 : ts);
+    const double rts = 1.0 / ts;
     uint8_t* srow = srows + (int64_t)row * srs;
     uint8_t* erow = rows + (int64_t)row * rs;
 
     for (int g0 = 0; g0 < NG; g0 += 64) {                // uniform: every lane shuffles
         const int g = g0 + lane;
         const bool ok = g < NG;
-        double xv[16];
-        double amax = 0.0;
+        // the search without divisions first (see near_error), on x * (1 / ts) for x / ts
+        double xq[16];
+        const double amax = load_block(x + 16 * g, ok, xq) / ts;
 #pragma unroll
-        for (int i = 0; i < 16; ++i) {
-            xv[i] = ok ? (double)x[16 * g + i] / ts : 0.0;
-            amax = fmax(amax, fabs(xv[i]));
-        }
-        double best_s = 1.0, best_e = 0.0;
+        for (int i = 0; i < 16; ++i) xq[i] *= rts;
+        auto at = [&](int i) { return ok ? (double)x[16 * g + i] : 0.0; };    // read again: seldom used
+        auto scale = [&](int c) {
+            const double s = e4m3_val(e4m3_rne(amax * sr.f[c] / 6.0));
+            return amax == 0.0 || s == 0.0 ? 1.0 : s;
+        };
+        const double X = sum_squares(xq), inf = __builtin_inf();
+        const bool plain = X < inf && amax < inf && ts > 0.0;         // (no NaN, no infinity)
+        double best_s = 0.0, best_e = inf, next_e = inf, last = 0.0, s1 = 0.0;
+#pragma unroll 1
         for (int c = 0; c < 13; ++c) {
-            double s = e4m3_val(e4m3_rne(amax * sr.f[c] / 6.0));
-            if (amax == 0.0 || s == 0.0) s = 1.0;
-            double p[8];
-#pragma unroll
-            for (int i = 0; i < 16; ++i) {
-                const double v = xv[i];
-                const double sg = v > 0.0 ? 1.0 : (v < 0.0 ? -1.0 : 0.0);
-                const double q = sg * mag[e2m1_code(v / s)] * s;
-                const double e = (q - v) * (q - v);
-                if (i < 8) p[i] = e;
-                else p[i & 7] = p[i & 7] + e;
-            }
-            const double err = ((p[0] + p[1]) + (p[2] + p[3])) + ((p[4] + p[5]) + (p[6] + p[7]));
-            if (c == 0 || err < best_e) { best_e = err; best_s = s; }
+            const double s = scale(c);
+            if (s == last) continue;
+            last = s;
+            s1 = fmax(s1, s);
+            const double E = near_error<true>(xq, s);
+            if (E < best_e) { next_e = best_e; best_e = E; best_s = s; }
+            else next_e = fmin(next_e, E);
         }
-        uint32_t word[2] = {0, 0};
+        const double reach = best_e + SEARCH_TOL * (best_e + X + 64.0 * (s1 * s1));
+        if (!(plain && next_e > reach)) {
+            bool first = true;
+            last = 0.0;
+#pragma unroll 1
+            for (int c = 0; c < 13; ++c) {
+                const double s = scale(c);
+                if (s == last) continue;
+                last = s;
+                if (plain && near_error<true>(xq, s) > reach) continue;
+                double p[8] = {0.0, 0.0, 0.0, 0.0, 0.0, 0.0, 0.0, 0.0};      // (0 + e is e)
+#pragma unroll 1
+                for (int i0 = 0; i0 < 16; i0 += 8) {
 #pragma unroll
-        for (int i = 0; i < 16; ++i) {
-            const double v = xv[i];
-            const double sg = v > 0.0 ? 1.0 : (v < 0.0 ? -1.0 : 0.0);
-            const double gq = (sg * mag[e2m1_code(v / best_s)] * best_s) / best_s;
-            const int mg = e2m1_code(gq);
-            const uint32_t code = (uint32_t)(mg | ((signbit(gq) && mg != 0) ? 8 : 0));
-            word[i >> 3] |= code << (4 * (i & 7));
+                    for (int i = 0; i < 8; ++i) {
+                        const double v = at(i0 + i) / ts;
+                        const double sg = v > 0.0 ? 1.0 : (v < 0.0 ? -1.0 : 0.0);
+                        const double q = sg * mag[e2m1_code(v / s)] * s;
+                        p[i] = p[i] + (q - v) * (q - v);
+                    }
+                }
+                const double err = ((p[0] + p[1]) + (p[2] + p[3])) + ((p[4] + p[5]) + (p[6] + p[7]));
+                if (first || err < best_e) { best_e = err; best_s = s; }
+                first = false;
+            }
+        }
+        uint32_t word[2];
+        if (!(near_codes<true>(xq, best_s, word) && plain)) {
+#pragma unroll 1
+            for (int w = 0; w < 2; ++w) {
+                uint32_t u = 0;
+#pragma unroll
+                for (int i = 0; i < 8; ++i) {
+                    const double v = at(8 * w + i) / ts;
+                    const double sg = v > 0.0 ? 1.0 : (v < 0.0 ? -1.0 : 0.0);
+                    const double gq = (sg * mag[e2m1_code(v / best_s)] * best_s) / best_s;
+                    const int mg = e2m1_code(gq);
+                    u |= (uint32_t)(mg | ((signbit(gq) && mg != 0) ? 8 : 0)) << (4 * i);
+                }
+                if (w == 0) word[0] = u;
+                else word[1] = u;
+            }
         }
         if (ok) *reinterpret_cast<uint2*>(erow + 8 * g) = make_uint2(word[0], word[1]);
         // the block's eight E4M3 bytes, assembled by its first lane
