@@ -103,16 +103,26 @@ def call(name: str, *args) -> None:
         raise OtpuError(rc, load().otpu_last_error().decode())
 
 
+_T = None
+
+
 def torch():
-    import torch as T
-    if not T.cuda.is_available():
-        raise RuntimeError("opentpu_amd needs a GPU (HIP device); none is visible")
-    return T
+    global _T
+    if _T is None:
+        import torch as T
+        if not T.cuda.is_available():
+            raise RuntimeError("opentpu_amd needs a GPU (HIP device); none is visible")
+        _T = T
+        for k, v in _NP2T.items():
+            _DTYPES[k] = _DTYPES[np.dtype(k)] = getattr(T, v)
+    return _T
 
 
 def stream():
-    """The current torch stream of the current device, as a hipStream_t."""
-    return C.c_void_p(torch().cuda.current_stream().cuda_stream)
+    """The current torch stream of the current device, as a hipStream_t (a few tenths of a us;
+    torch.cuda.current_stream() builds a Stream object, 3 us)."""
+    T = _T or torch()
+    return C.c_void_p(T._C._cuda_getCurrentRawStream(T.cuda.current_device()))
 
 
 def ptr(t):
@@ -121,12 +131,18 @@ def ptr(t):
 
 _NP2T = {np.float32: "float32", np.int8: "int8", np.uint8: "uint8", np.int64: "int64",
          np.int32: "int32", np.uint64: "uint64", np.float64: "float64"}
+_DTYPES = {}                                    # numpy scalar type or dtype -> torch dtype, once torch is loaded
+
+
+def _dtype(dtype):
+    t = _DTYPES.get(dtype)
+    return t if t is not None else _DTYPES[np.dtype(dtype).type]
 
 
 def dev(x, dtype):
     """A contiguous device tensor of dtype (a numpy dtype) from a numpy array or a tensor."""
-    T = torch()
-    tdt = getattr(T, _NP2T[np.dtype(dtype).type])
+    T = _T or torch()
+    tdt = _dtype(dtype)
     if isinstance(x, T.Tensor):
         if x.dtype != tdt:
             if tdt == T.uint8 and x.dtype == T.int8 or tdt == T.int8 and x.dtype == T.uint8:
@@ -144,13 +160,13 @@ def dev(x, dtype):
 
 
 def empty(shape, dtype):
-    T = torch()
-    return T.empty(shape, dtype=getattr(T, _NP2T[np.dtype(dtype).type]), device="cuda")
+    T = _T or torch()
+    return T.empty(shape, dtype=_dtype(dtype), device="cuda")
 
 
 def zeros(shape, dtype):
-    T = torch()
-    return T.zeros(shape, dtype=getattr(T, _NP2T[np.dtype(dtype).type]), device="cuda")
+    T = _T or torch()
+    return T.zeros(shape, dtype=_dtype(dtype), device="cuda")
 
 
 def is_numpy(x) -> bool:

@@ -149,22 +149,36 @@ class QWeight:
         return QWeight(X.dev(rows, np.uint8), X.dev(srows, np.uint8), fmt, K, rsc)
 
 
+def _check_ranges(ranges, K: int) -> list:
+    ranges = [K] if ranges is None else list(ranges)
+    if sum(ranges) != K or any(r % D for r in ranges):
+        raise ValueError(f"quantize_ranges: ranges {ranges} over {K} columns")
+    return ranges
+
+
+def _qact_equal(xd, ranges, row_mode: bool, q: int, Sa: int, da: int, stream) -> None:
+    """QACT of equal ranges into packed buffers (their addresses), one launch."""
+    M, K = xd.shape
+    fl = X.Q_ROW if row_mode else 0
+    if len(ranges) > 1:
+        X.call("otpu_qact_ranges", xd.data_ptr(), None, M, K, K, ranges[0], 32, fl, None, None, q, K, Sa, da, K // 32, stream)
+    else:
+        X.call("otpu_qact", xd.data_ptr(), M, K, K, 32, fl, None, None, q, K, Sa, da, K // 32, None, 0, stream)
+
+
 def quantize_ranges(x, ranges=None, row_mode: bool = False):
     """QACT of x [M, K] in column ranges (widths summing to K, each a multiple of 128; default
     one range): the int8 operand [M, K], Sa per range [n_ranges, M], da [M, K/32]."""
     xd = X.dev(x, np.float32)
     M, K = xd.shape
-    ranges = [K] if ranges is None else list(ranges)
-    if sum(ranges) != K or any(r % D for r in ranges):
-        raise ValueError(f"quantize_ranges: ranges {ranges} over {K} columns")
+    ranges = _check_ranges(ranges, K)
     q = X.empty((M, K), np.int8)
     da = X.empty((M, K // 32), np.uint8)
     Sa = X.empty((len(ranges), M), np.float32)
-    flags = X.Q_ROW if row_mode else 0
-    if len(ranges) > 1 and min(ranges) == max(ranges):    # equal ranges: one launch
-        X.call("otpu_qact_ranges", X.ptr(xd), None, M, K, K, ranges[0], 32, flags, None, None, X.ptr(q), K, X.ptr(Sa),
-               X.ptr(da), K // 32, X.stream())
+    if min(ranges) == max(ranges):
+        _qact_equal(xd, ranges, row_mode, q.data_ptr(), Sa.data_ptr(), da.data_ptr(), X.stream())
         return q, Sa, da, ranges
+    flags = X.Q_ROW if row_mode else 0
     c0 = 0
     for i, w in enumerate(ranges):
         xs = xd[:, c0:c0 + w]
@@ -209,6 +223,18 @@ def _dot_row(x, w: QWeight, ranges, out) -> bool:
     return True
 
 
+def _scratch(*sizes):
+    """The addresses of buffers of these sizes (bytes, each aligned to 256) and the allocation that
+    holds them, to be kept until the launches that use them are queued."""
+    offs, n = [], 0
+    for b in sizes:
+        offs.append(n)
+        n += (b + 255) & ~255
+    t = X.empty((n,), np.uint8)
+    p = t.data_ptr()
+    return *(p + o for o in offs), t
+
+
 def dot(x, w: QWeight, acc=None, out=None, ranges=None, row_mode: bool = False, rowmax: bool = False,
         acc_scale=None):
     """x [M, K] (fp32, quantized here, or a (q, Sa, da, ranges) operand from quantize_ranges)
@@ -236,22 +262,32 @@ def dot(x, w: QWeight, acc=None, out=None, ranges=None, row_mode: bool = False, 
                 y = out if out is not None else X.empty((1, N), np.float32)
                 if _dot_row(xd, w, rl, y):
                     return X.host(y) if numpy_in else y
-        q, Sa, da, ranges = quantize_ranges(xd, ranges, row_mode)
+        ranges = _check_ranges(ranges, K)
+        M = xd.shape[0]
     else:
         q, Sa, da, ranges = x
-    M, K = q.shape
-    if K != w.K:
-        raise ValueError(f"dot: K mismatch {K} vs {w.K}")
-    y = X.dev(acc, np.float32) if acc is not None else (out if out is not None else X.empty((M, N), np.float32))
+        M, K = q.shape
+        if K != w.K:
+            raise ValueError(f"dot: K mismatch {K} vs {w.K}")
     unit = w.srows is None
-    al = X.dev(acc_scale, np.float32) if acc_scale is not None else None
     chunk = D if w.fmt == "int8" else 2 * D
     width = ranges[0]
-    if not rowmax and (len(ranges) == 1 or (min(ranges) == max(ranges) and width % chunk == 0)):
-        act = X.ACT_ANY if operand else (X.ACT_ROW if row_mode else X.ACT_MX)
-        X.call("otpu_mm_dot", q.data_ptr(), K, Sa.data_ptr(), da.data_ptr(), K // 32, M, K, width, w.rows.data_ptr(),
-               w.rows.shape[1], 0 if unit else w.srows.data_ptr(), 0 if unit else w.srows.shape[1], N, X.FMT[w.fmt],
-               _flags(unit, w.rsc, acc is not None, al is not None), 0, act, X.ptr(al), y.data_ptr(), N, X.stream())
+    one = not rowmax and (len(ranges) == 1 or (min(ranges) == max(ranges) and width % chunk == 0))
+    if not operand and not one:
+        q, Sa, da, ranges = quantize_ranges(xd, ranges, row_mode)
+    y = X.dev(acc, np.float32) if acc is not None else (out if out is not None else X.empty((M, N), np.float32))
+    al = X.dev(acc_scale, np.float32) if acc_scale is not None else None
+    if one:
+        s = X.stream()
+        if operand:
+            qp, Sp, dp, act = q.data_ptr(), Sa.data_ptr(), da.data_ptr(), X.ACT_ANY
+        else:                                             # the operand's three parts in one allocation
+            qp, Sp, dp, _scr = _scratch(M * K, 4 * M * len(ranges), M * (K // 32))
+            act = X.ACT_ROW if row_mode else X.ACT_MX
+            _qact_equal(xd, ranges, row_mode, qp, Sp, dp, s)
+        X.call("otpu_mm_dot", qp, K, Sp, dp, K // 32, M, K, width, w.rows.data_ptr(), w.rows.shape[1],
+               0 if unit else w.srows.data_ptr(), 0 if unit else w.srows.shape[1], N, X.FMT[w.fmt],
+               _flags(unit, w.rsc, acc is not None, al is not None), 0, act, X.ptr(al), y.data_ptr(), N, s)
         return X.host(y) if numpy_in else y
     bpb = D if w.fmt == "int8" else D // 2
     rm = X.empty((M,), np.float32) if rowmax else None
