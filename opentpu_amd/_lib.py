@@ -112,9 +112,9 @@ def torch():
         import torch as T
         if not T.cuda.is_available():
             raise RuntimeError("opentpu_amd needs a GPU (HIP device); none is visible")
-        _T = T
         for k, v in _NP2T.items():
             _DTYPES[k] = _DTYPES[np.dtype(k)] = getattr(T, v)
+        _T = T                                  # last: another thread that sees it finds the dtypes
     return _T
 
 

@@ -273,6 +273,9 @@ def dot(x, w: QWeight, acc=None, out=None, ranges=None, row_mode: bool = False, 
     chunk = D if w.fmt == "int8" else 2 * D
     width = ranges[0]
     one = not rowmax and (len(ranges) == 1 or (min(ranges) == max(ranges) and width % chunk == 0))
+    if operand and one:                                   # scales of other strides, offsets of odd addresses: a launch a range
+        one = da.data_ptr() % 4 == 0 and (len(ranges) == 1 or (
+            isinstance(Sa, X.torch().Tensor) and Sa.is_contiguous() and Sa.shape[1] == M))
     if not operand and not one:
         q, Sa, da, ranges = quantize_ranges(xd, ranges, row_mode)
     y = X.dev(acc, np.float32) if acc is not None else (out if out is not None else X.empty((M, N), np.float32))
@@ -280,7 +283,7 @@ def dot(x, w: QWeight, acc=None, out=None, ranges=None, row_mode: bool = False, 
     if one:
         s = X.stream()
         if operand:
-            qp, Sp, dp, act = q.data_ptr(), Sa.data_ptr(), da.data_ptr(), X.ACT_ANY
+            qp, Sp, dp, act = q.data_ptr(), Sa[0].data_ptr(), da.data_ptr(), X.ACT_ANY
         else:                                             # the operand's three parts in one allocation
             qp, Sp, dp, _scr = _scratch(M * K, 4 * M * len(ranges), M * (K // 32))
             act = X.ACT_ROW if row_mode else X.ACT_MX

@@ -161,3 +161,22 @@ def test_mm_dot_refuses(X):
     for kw in ({"width": 128}, {"width": 300}, {"width": 512, "act": 3}, {"width": 512, "flags": MM.RMAX}):
         with pytest.raises(X.OtpuError):
             mm_dot(X, q, Sa, da, rows, srows, "int4", 512, kw["width"], kw.get("flags", 0), act=kw.get("act", 0))
+
+
+@pytest.mark.parametrize("fmt,ranges", [("int4", [256, 256, 256]), ("int8", [768])])
+def test_dot_of_an_operands_rows(X, fmt, ranges):
+    """Rows of a longer operand: Sa's strides are those of the whole; offsets from an odd address."""
+    import torch
+    from opentpu_amd import mxu
+    rng = np.random.default_rng(7)
+    N, K = 70, 768
+    _, _, _, rows, srows, _ = operands(rng, 1, N, K, fmt, "spread", "mx")
+    w = mxu.QWeight.from_packed(rows, srows, fmt, K)
+    x = torch.from_numpy(rng.standard_normal((20, K)).astype(np.float32)).cuda()
+    q, Sa, da, rg = mxu.quantize_ranges(x, ranges)
+    say("dot of rows 4..16", fmt, ranges)
+    want = X.host(mxu.dot(x[4:17].contiguous(), w, ranges=ranges))
+    assert same_bits(X.host(mxu.dot((q[4:17], Sa[:, 4:17], da[4:17], rg), w)), want)
+    odd = torch.empty((13 * (K // 32) + 1,), dtype=torch.uint8, device="cuda")[1:].view(13, K // 32)
+    odd.copy_(da[4:17])
+    assert same_bits(X.host(mxu.dot((q[4:17], Sa[:, 4:17].contiguous(), odd, rg), w)), want)
