@@ -15,9 +15,9 @@ int otpu_prefill_try(const int8_t* q, int64_t ldq, const float* Sa, const uint8_
     a.k0 = (flags & (OTPU_UNIT | OTPU_RSC)) ? 0 : k0;
     a.alpha = alpha; a.out = out; a.ors = ors; a.ranges = ranges;
     // 64 rows a tile where that still makes two workgroups a CU, else 32 (int4 2000 x 1024 x 4096: 50
-    // against 54 us; 512 x 2048 x 1024: 30 against 22; nvfp4's ranges at 64 rows spill registers)
+    // against 54 us; 512 x 2048 x 1024: 30 against 22; nvfp4 1999 x 6144 x 2048 in ranges of 768: 222 against 280)
     const int64_t t64 = (int64_t)((M + 63) / 64) * ((N + 127) / 128);
-    const int ms = t64 >= 2 * otpu_cu_count() && !(fmt == OTPU_NVFP4 && ranges > 1) ? 2 : 1;
+    const int ms = t64 >= 2 * otpu_cu_count() ? 2 : 1;
     a.tiles_m = (M + 32 * ms - 1) / (32 * ms);
     a.tiles_n = (N + 127) / 128;
     a.vec4 = ((uintptr_t)out % 16 == 0) && (ors % 4 == 0);

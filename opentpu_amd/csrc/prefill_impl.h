@@ -3,7 +3,7 @@
 // (opentpu/compiler.py:2686-2720).
 //
 // One v_mfma_i32_32x32x32_i8 is one 32-group of 32 weight rows x 32 activation rows (nvfp4: two of
-// them, its 16-groups), and its int32 sums are the groups' integer dot products c whatever
+// K 16, its 16-groups), and its int32 sums are the groups' integer dot products c whatever
 // offsets the operands carry.  The terms m c 2^(W - dw - da) are added on the VALU: one walk of K
 // serves every activation offset and weight multiplier.  (The same GEMM with the scales folded into
 // int8 operand planes multiplies two planes of the weights once for each activation offset present,
@@ -24,11 +24,15 @@
 #pragma once
 #include "prefill_args.h"
 
+#include <type_traits>
+
 namespace otpu {
 namespace pf {
 
 typedef int v4i __attribute__((ext_vector_type(4)));
 typedef int v16i __attribute__((ext_vector_type(16)));
+typedef unsigned short us2 __attribute__((ext_vector_type(2)));
+typedef short s2 __attribute__((ext_vector_type(2)));
 
 // the kernel's lambdas are all inlined: a call would put its sums in memory
 #define INL __attribute__((always_inline))
@@ -117,6 +121,7 @@ __device__ __forceinline__ void prefill_tile(const Args& p, int8_t* ring, int m0
     using T = Tile<FMT, MS, MH>;
     constexpr bool I8 = T::I8, NV = T::NV;
     constexpr int W = F::W, NST = T::NST, MW = T::MW;
+    constexpr bool NEG = FMT == OTPU_INT4 && !RANGED;     // weights and multipliers negated (dots)
     const float* const sSw = reinterpret_cast<const float*>(ring + T::SCALE);
 
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -184,12 +189,14 @@ __device__ __forceinline__ void prefill_tile(const Args& p, int8_t* ring, int m0
     int ew = 0, sd = 0;                                   // the unit: 2^(W - ew - sd)
     bool wide = false;                                    // the unit: 1
     uint32_t bound = 0;                                   // of |acc|
+    bool low = true;                                      // every hi 0
     auto clear = [&]() INL {
 #pragma unroll
         for (int i = 0; i < MS; ++i)
 #pragma unroll
             for (int t = 0; t < 16; ++t) acc[i][t] = hi[i][t] = 0;
         bound = 0;
+        low = true;
         if (wide) ew = sd = 0;                            // (ranges: the next one starts at this one's unit)
         wide = false;
     };
@@ -203,6 +210,7 @@ __device__ __forceinline__ void prefill_tile(const Args& p, int8_t* ring, int m0
                 acc[i][t] &= 0xFFFF;
             }
         bound = 65536;
+        low = false;
     };
     auto finer = [&](int up) INL {                        // to a unit 2^up finer (up <= 16)
         if (((uint64_t)bound << up) >= (1ull << 31)) {
@@ -230,11 +238,17 @@ __device__ __forceinline__ void prefill_tile(const Args& p, int8_t* ring, int m0
     // output t of row tile i: row mrow(i), column ncol(t)
     auto mrow = [&](int i) INL { return m0 + 32 * (MS * mh + i) + r32; };
     auto ncol = [&](int t) INL { return n0 + 32 * wid + 8 * (t >> 2) + 4 * h + (t & 3); };
-    auto value = [&](int i, int t, float sa) INL {
-        const double v = ((double)hi[i][t] * 65536.0 + (double)acc[i][t]) *
-                         __hiloint2double((1023 + (wide ? 0 : W - ew - sd)) << 20, 0);
+    // the sum's fp32 value times the scales: a sum of one int32 is rounded to fp32 as it is (then a power
+    // of two >= 1), one with an upper part goes through a double
+    auto value = [&](int i, int t, float sa, auto one) INL {
+        float v;
+        if constexpr (decltype(one)::value)
+            v = (float)acc[i][t] * bitsf((uint32_t)(127 + W - ew - sd) << 23);
+        else
+            v = (float)(((double)hi[i][t] * 65536.0 + (double)acc[i][t]) *
+                        __hiloint2double((1023 + (wide ? 0 : W - ew - sd)) << 20, 0));
         const float sw = (p.flags & OTPU_UNIT) ? 1.0f : ftz(sSw[32 * wid + 8 * (t >> 2) + 4 * h + (t & 3)]);
-        return fmul_f(fmul_f((float)v, sw), sa);
+        return fmul_f(fmul_f(v, sw), sa);
     };
     auto scale_m = [&](int i, int r) INL { return fmul(p.Sa[(int64_t)r * p.M + min(mrow(i), p.M - 1)], pow2f(-W)); };
     auto first = [&](float v, int m, int n) INL {             // joins the old output as a call's first MM does
@@ -245,7 +259,9 @@ __device__ __forceinline__ void prefill_tile(const Args& p, int8_t* ring, int m0
     };
 
     uint32_t tp[2], tn8[2];
-    if (FMT == OTPU_INT4) {
+    if (NEG) {
+        tp[0] = 0xFDFEFF00u; tp[1] = 0xF9FAFBFCu; tn8[0] = 0x05060708u; tn8[1] = 0x01020304u;
+    } else if (FMT == OTPU_INT4) {
         tp[0] = 0x03020100u; tp[1] = 0x07060504u; tn8[0] = 0xFBFAF9F8u; tn8[1] = 0xFFFEFDFCu;
     } else {                                              // twice the E2M1 values
         tp[0] = 0x03020100u; tp[1] = 0x0C080604u; tn8[0] = 0xFDFEFF00u; tn8[1] = 0xF4F8FAFCu;
@@ -319,7 +335,8 @@ __device__ __forceinline__ void prefill_tile(const Args& p, int8_t* ring, int m0
         } else if constexpr (!I8) {
             const uint32_t six = plain ? 0x01041041u : own >> 8;
             const uint32_t two = h ? six >> 12 : six;     // half h of the wave: groups 2 h, 2 h + 1
-            sMul[h][r32] = ((two & 63u) | ((two & (63u << 6)) << 10)) << (((uint32_t)ew - dw) & 31u);
+            const uint32_t m2 = ((two & 63u) | ((two & (63u << 6)) << 10)) << (((uint32_t)ew - dw) & 31u);
+            sMul[h][r32] = NEG ? __builtin_bit_cast(uint32_t, (us2)0 - __builtin_bit_cast(us2, m2)) : m2;
         }
     };
     // the unit made fine enough for a block of offsets d, its sums' bound counted
@@ -339,6 +356,7 @@ __device__ __forceinline__ void prefill_tile(const Args& p, int8_t* ring, int m0
                 if (nsd + new_ > F::SMAX) {
                     finer(W - ew - sd);
                     wide = true;
+                    low = false;
                 } else {
                     finer(nsd + new_ - ew - sd);
                     sd = nsd;
@@ -357,29 +375,21 @@ __device__ __forceinline__ void prefill_tile(const Args& p, int8_t* ring, int m0
     // use otherwise).  Running the pipeline on across blocks measured slower (int8 184 -> 198 us at
     // 2000 x 2048 x 12288): the two waves a SIMD holds are bound by their own issue. ----
     constexpr int NP = 4 * MS;                            // pairs a block
-    auto pairs = [&]() INL {
-        uint32_t mw[I8 ? 1 : 16];
-        auto mults = [&](int k) INL {                     // the 16 rows' words k: groups 2 k, 2 k + 1 (nvfp4: 16-groups)
-            if constexpr (!I8) {
+    uint32_t mw[I8 ? 1 : 16];
+    auto mults = [&](int k) INL {                         // the 16 rows' words k: groups 2 k, 2 k + 1 (nvfp4: 16-groups)
+        if constexpr (!I8) {
 #pragma unroll
-                for (int q = 0; q < 4; ++q) {
-                    const uint4 x = *reinterpret_cast<const uint4*>(&sMul[k][8 * q + 4 * h]);
-                    mw[4 * q] = x.x; mw[4 * q + 1] = x.y; mw[4 * q + 2] = x.z; mw[4 * q + 3] = x.w;
-                }
+            for (int q = 0; q < 4; ++q) {
+                const uint4 x = *reinterpret_cast<const uint4*>(&sMul[k][8 * q + 4 * h]);
+                mw[4 * q] = x.x; mw[4 * q + 1] = x.y; mw[4 * q + 2] = x.z; mw[4 * q + 3] = x.w;
             }
-        };
-        v16i c[2], c1[NV ? 2 : 1];
+        }
+    };
+    auto pairs = [&]() INL {
+        v16i c[2];
         v4i w = weights(cur, 0), a = acts(cur, 0, 0);
         mults(0);
-        auto product = [&](int j) INL {
-            if constexpr (NV) {                           // elements 0-15 are the wave's first half
-                const int k = h ? 0 : -1;
-                c[j & 1] = __builtin_amdgcn_mfma_i32_32x32x32_i8(w & k, a, zero, 0, 0, 0);
-                c1[j & 1] = __builtin_amdgcn_mfma_i32_32x32x32_i8(w & ~k, a, zero, 0, 0, 0);
-            } else {
-                c[j & 1] = __builtin_amdgcn_mfma_i32_32x32x32_i8(w, a, zero, 0, 0, 0);
-            }
-        };
+        auto product = [&](int j) INL { c[j & 1] = __builtin_amdgcn_mfma_i32_32x32x32_i8(w, a, zero, 0, 0, 0); };
         product(0);
         a = acts(cur, 1 % MS, 1 / MS);
         if (MS == 1) w = weights(cur, 1);
@@ -398,12 +408,79 @@ __device__ __forceinline__ void prefill_tile(const Args& p, int8_t* ring, int m0
             for (int t = 0; t < 16; ++t) {
                 int v;
                 if constexpr (I8) v = c[j & 1][t];
-                else if constexpr (NV)
-                    v = __mul24(c[j & 1][t], (int)(mw[t] & 0xFFFFu)) + __mul24(c1[j & 1][t], (int)(mw[t] >> 16));
                 else v = __mul24(c[j & 1][t], (int)(g & 1 ? mw[t] >> 16 : mw[t] & 0xFFFFu));
                 acc[i][t] += v << sh;
             }
             if (j + 1 < NP && (j + 1) % (NP / MW) == 0) mults((j + 1) / (NP / MW));
+        }
+    };
+    // int4 and nvfp4: their group products fit 16 bits with any int8 activations (nvfp4: 16 128 12; int4:
+    // -32 127 8 .. 32 128 8, the negated weights' -32768 .. 32512), so the terms of two groups are one
+    // v_dot2: pack the products, shift the two multipliers by the activation's offsets, multiply-add
+    // both.  The products of unit j + 1 run behind the sums of unit j, in the registers its packing
+    // freed: 16 fewer than two sets (nvfp4's ranges at 64 rows a tile spill 5 registers, not 104).
+    // Measured (us, QACT in; a multiply and a shift-add a group -> this): int4 1999 x 2048 x 12288 239 ->
+    // 233; nvfp4 (its 16-groups as K 16 products, no masked lanes) 337 -> 328, 1999 x 6144 x 2048 in
+    // ranges of 768 280 -> 222.  int4's ranges keep the other form (64 rows a tile: 169 against 175).
+    auto dots = [&]() INL {
+        constexpr int NU = MW * MS;                       // units (multiplier word k, row tile i)
+        // operands: int4 two groups', nvfp4 one group's two 16-groups (8 elements a lane, K 16 products)
+        using Op = std::conditional_t<NV, long, v4i>;
+        Op w[2], a[2];
+        auto fetch = [&](int j) INL {
+            const int k = j / MS, r = 32 * (MS * mh + j % MS) + r32;
+            if constexpr (NV) {
+                if (j % MS == 0) {
+                    const uint32_t* B = reinterpret_cast<const uint32_t*>(cur + T::AB + r0 * 64 + 16 * swz4(r0, k)) + h;
+#pragma unroll
+                    for (int e = 0; e < 2; ++e) {
+                        uint32_t lo, up;
+                        lookup8(B[2 * e], tp, tn8, lo, up);
+                        w[e] = (long)((uint64_t)up << 32 | lo);
+                    }
+                }
+#pragma unroll
+                for (int e = 0; e < 2; ++e) a[e] = *reinterpret_cast<const long*>(cur + r * 128 + 16 * swz8(r, 2 * k + e) + 8 * h);
+            } else {
+#pragma unroll
+                for (int e = 0; e < 2; ++e) {
+                    if (j % MS == 0) w[e] = weights(cur, 2 * k + e);
+                    a[e] = acts(cur, j % MS, 2 * k + e);
+                }
+            }
+        };
+        v16i c0, c1;
+        auto product = [&]() INL {
+            if constexpr (NV) {
+                c0 = __builtin_amdgcn_mfma_i32_32x32x16_i8(w[0], a[0], zero, 0, 0, 0);
+                c1 = __builtin_amdgcn_mfma_i32_32x32x16_i8(w[1], a[1], zero, 0, 0, 0);
+            } else {
+                c0 = __builtin_amdgcn_mfma_i32_32x32x32_i8(w[0], a[0], zero, 0, 0, 0);
+                c1 = __builtin_amdgcn_mfma_i32_32x32x32_i8(w[1], a[1], zero, 0, 0, 0);
+            }
+        };
+        fetch(0);
+        mults(0);
+        product();
+        fetch(1);
+#pragma unroll
+        for (int j = 0; j < NU; ++j) {
+            const int k = j / MS, i = j % MS;
+            uint32_t c[16];                               // the low halves of both products
+#pragma unroll
+            for (int t = 0; t < 16; ++t) c[t] = __builtin_amdgcn_perm((uint32_t)c1[t], (uint32_t)c0[t], 0x05040100u);
+            __builtin_amdgcn_sched_barrier(0);
+            if (j + 1 < NU) product();
+            if (j + 2 < NU) fetch(j + 2);
+            __builtin_amdgcn_sched_barrier(0);
+            const uint32_t d0 = (da[i] >> (NV ? 8 * k : 16 * k)) & 0xFFu, d1 = NV ? d0 : (da[i] >> (16 * k + 8)) & 0xFFu;
+            const us2 sh = {(unsigned short)((uint32_t)sd - d0), (unsigned short)((uint32_t)sd - d1)};
+#pragma unroll
+            for (int t = 0; t < 16; ++t) {
+                const us2 m = __builtin_bit_cast(us2, mw[t]) << sh;
+                acc[i][t] = __builtin_amdgcn_sdot2(__builtin_bit_cast(s2, c[t]), __builtin_bit_cast(s2, m), acc[i][t], false);
+            }
+            if (j + 1 < NU && (j + 1) % MS == 0) mults((j + 1) / MS);
         }
     };
 
@@ -420,7 +497,8 @@ __device__ __forceinline__ void prefill_tile(const Args& p, int8_t* ring, int m0
 
         const bool shifted = I8 && __any(dw != 0);        // (uniform)
         if (!wide && !shifted && !(I8 && sd + ew == 0)) {
-            pairs();
+            if constexpr (NV || NEG) dots();
+            else pairs();
         } else {
             const uint32_t* X = words(cur);
             if (I8 && !wide && !shifted) {                // no offset so far: the MFMA's own sums
@@ -477,6 +555,7 @@ __device__ __forceinline__ void prefill_tile(const Args& p, int8_t* ring, int m0
                                         wd = (int)(word & 0xFFu);
                                     }
                                 }
+                                if (NEG) m = -m;
                                 const int s = W - wd - d;
                                 const int64_t v = s >= 0 ? (int64_t)(x[t] * m) << (s & 31) : 0;
                                 acc[i][t] += (int)(v & 0xFFFF);
@@ -491,48 +570,56 @@ __device__ __forceinline__ void prefill_tile(const Args& p, int8_t* ring, int m0
         if constexpr (RANGED) {
             if ((kb + 1) % KR == 0) {
                 const int r = kb / KR;
+                auto fold = [&](auto one) INL {
 #pragma unroll
-                for (int i = 0; i < MS; ++i) {
-                    const float sa = scale_m(i, r);
+                    for (int i = 0; i < MS; ++i) {
+                        const float sa = scale_m(i, r);
 #pragma unroll
-                    for (int t = 0; t < 16; ++t) {
-                        const float v = value(i, t, sa);
-                        if (r) y[i][t] = fadd(y[i][t], v);
-                        else y[i][t] = mrow(i) < p.M && ncol(t) < p.N ? first(v, mrow(i), ncol(t)) : v;
+                        for (int t = 0; t < 16; ++t) {
+                            const float v = value(i, t, sa, one);
+                            if (r) y[i][t] = fadd(y[i][t], v);
+                            else y[i][t] = mrow(i) < p.M && ncol(t) < p.N ? first(v, mrow(i), ncol(t)) : v;
+                        }
                     }
-                }
+                };
+                if (low) fold(std::true_type());
+                else fold(std::false_type());
                 clear();
             }
         }
     }
     // ---- the outputs: 4 adjacent columns a store ----
+    auto outputs = [&](auto one) INL {
 #pragma unroll
-    for (int i = 0; i < MS; ++i) {
-        const int m = mrow(i);
-        if (m >= p.M) continue;
-        const float sa = RANGED ? 0.0f : scale_m(i, 0);
+        for (int i = 0; i < MS; ++i) {
+            const int m = mrow(i);
+            if (m >= p.M) continue;
+            const float sa = RANGED ? 0.0f : scale_m(i, 0);
 #pragma unroll
-        for (int q = 0; q < 4; ++q) {
-            const int n = ncol(4 * q);
-            float* o = p.out + (int64_t)m * p.ors + n;
-            float v[4];
+            for (int q = 0; q < 4; ++q) {
+                const int n = ncol(4 * q);
+                float* o = p.out + (int64_t)m * p.ors + n;
+                float v[4];
 #pragma unroll
-            for (int u = 0; u < 4; ++u) {
-                if constexpr (RANGED) v[u] = y[i][4 * q + u];
-                else v[u] = value(i, 4 * q + u, sa);
-            }
-            if (p.vec4 && n + 3 < p.N) {
-                if (!RANGED)
+                for (int u = 0; u < 4; ++u) {
+                    if constexpr (RANGED) v[u] = y[i][4 * q + u];
+                    else v[u] = value(i, 4 * q + u, sa, one);
+                }
+                if (p.vec4 && n + 3 < p.N) {
+                    if (!RANGED)
 #pragma unroll
-                    for (int u = 0; u < 4; ++u) v[u] = first(v[u], m, n + u);
-                *reinterpret_cast<float4*>(o) = make_float4(v[0], v[1], v[2], v[3]);
-            } else {
+                        for (int u = 0; u < 4; ++u) v[u] = first(v[u], m, n + u);
+                    *reinterpret_cast<float4*>(o) = make_float4(v[0], v[1], v[2], v[3]);
+                } else {
 #pragma unroll
-                for (int u = 0; u < 4; ++u)
-                    if (n + u < p.N) o[u] = RANGED ? v[u] : first(v[u], m, n + u);
+                    for (int u = 0; u < 4; ++u)
+                        if (n + u < p.N) o[u] = RANGED ? v[u] : first(v[u], m, n + u);
+                }
             }
         }
-    }
+    };
+    if (RANGED || low) outputs(std::true_type());
+    else outputs(std::false_type());
 }
 
 template <int FMT, int MS, bool RANGED>

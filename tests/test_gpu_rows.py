@@ -85,6 +85,25 @@ def test_prefill(X, M, N, K, act, fmt, wk, ak):
     assert same_bits(got, OC.mm(q, Sa, da, rows, srows, fmt, K, flags=fl))
 
 
+@pytest.mark.parametrize("fmt,lo,hi", [("int4", 0x88, 0x77), ("nvfp4", 0xFF, 0x77)])
+def test_prefill_largest_products(X, fmt, lo, hi):
+    """Group products at the ends of their range: activations -128 and 127 (any int8 may come as an
+    operand) on the largest weights of either sign, offsets 0 and 2."""
+    M, N, K = 100, 8100, 256
+    rng = np.random.default_rng(3)
+    _, _, _, rows, srows, _ = operands(rng, 1, N, K, fmt, "x4", "mx")
+    rows = rows.copy()
+    rows[0::2], rows[1::2] = lo, hi
+    q = np.where(np.arange(M) % 2, 127, -128).astype(np.int8)[:, None].repeat(K, 1)
+    Sa = np.full(M, 0.01, np.float32)
+    da = np.zeros((M, K // 32), np.uint8)
+    da[::3, ::2] = 2
+    say("prefill largest products", fmt)
+    got = mm_dot(X, q, Sa, da, rows, srows, fmt, K, K, act=2)
+    cut = np.ascontiguousarray
+    assert same_bits(got[:, :40], OC.mm(q, Sa, da, cut(rows[:40]), cut(srows[:40]), fmt, K))
+
+
 @pytest.mark.parametrize("fmt", ["int8", "int4", "nvfp4"])
 def test_prefill_long_sums(X, fmt):
     """Sums that leave int32 inside the walk: every product at its largest over K = 16384."""
