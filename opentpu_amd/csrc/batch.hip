@@ -20,7 +20,12 @@ int otpu_batch_try(const int8_t* q, int64_t ldq, const float* Sa, const uint8_t*
     int kwmax = 8;
     while (kwmax > parts) kwmax >>= 1;
     const int64_t want = 8 * (int64_t)otpu_cu_count();
-    int nsub = 4;
+    // 64 weight rows a wave tile, but 32 beside 32 activation rows where those spill (int8 101 registers,
+    // int4 41): us at 64 -> at 32, QACT in: int8 512 x 2048 x 1024 22.1 -> 18.3, 512 x 3072 x 1024 in ranges of 256
+    // 46.0 -> 31.9, 100 x 2048 x 6000 36.3 -> 29.1; nvfp4 29.6 -> 26.0, 61.7 -> 46.7, 49.9 -> 43.2; fp4's ranges 40.2
+    // -> 37.4, int4's 37.6 -> 36.4, but without ranges int4 100 x 2048 x 6000 31.7 -> 33.4, fp4 34.7 -> 34.8
+    const bool spills = fmt == OTPU_INT8 || fmt == OTPU_NVFP4 || ranges > 1;
+    int nsub = mt == 2 && spills ? 2 : 4;
     while (nsub > 1 && (int64_t)((N + 16 * nsub - 1) / (16 * nsub)) * tiles_m * kwmax < want) nsub >>= 1;
     int kw = 1;
     while (kw < kwmax && (int64_t)((N + 16 * nsub - 1) / (16 * nsub)) * tiles_m * kw < want) kw <<= 1;

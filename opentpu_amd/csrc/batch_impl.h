@@ -440,7 +440,7 @@ void launch_fmt(const Args& a, int nsub, int mt, hipStream_t s) {
     } else {
         if (nsub == 1) launch<FMT, 1, 2>(a, s);
         else if (nsub == 2) launch<FMT, 2, 2>(a, s);
-        else launch<FMT, 4, 2>(a, s);
+        else if constexpr (FMT == OTPU_INT4 || FMT == OTPU_FP4) launch<FMT, 4, 2>(a, s);   // (others: batch.hip's rule)
     }
 }
 
