@@ -112,13 +112,14 @@ static int check_mm(const char* who, const int8_t* q, int64_t ldq, const uint8_t
     return OTPU_OK;
 }
 
-// lanes per row: the team size in {64, 32, 16} that wastes the fewest lane pieces; a row of
-// more than 64 LMAX pieces takes teams of 64 with LMAX pieces a lane, walked in segments
-static void pick_team(int P, int* T, int* L, int* nseg = nullptr) {
+// lanes per row: the team size in {64, 32, 16} that wastes the fewest lane pieces, of those with at
+// most lmax pieces a lane; a row of more than 64 LMAX pieces takes teams of 64 with LMAX pieces a
+// lane, walked in segments
+static void pick_team(int P, int* T, int* L, int* nseg = nullptr, int lmax = LMAX) {
     int bt = 64, bl = (P + 63) / 64, bw = bl * 64 - P;
     for (int t = 32; t >= 16; t >>= 1) {
         int l = (P + t - 1) / t, w = l * t - P;
-        if (l <= LMAX && w < bw) { bt = t; bl = l; bw = w; }
+        if (l <= lmax && w < bw) { bt = t; bl = l; bw = w; }
     }
     if (bl == 7) bl = 8;                        // (no L = 7 instantiation: the eighth is masked)
     const int ns = bl > LMAX ? (bl + LMAX - 1) / LMAX : 1;
@@ -420,11 +421,10 @@ int fold_args(MMArgs* ap, int* Lp, const float* x, const float* xmul, const floa
     a.rscale = rscale; a.cscale = cscale;
     a.P = (K / 2) / 16;
     a.fold_c = width / 256;
-    int L = 1;
-    pick_team(a.P, &a.T, &L);
-    if (L > 4) return otpu_fail(OTPU_EINVAL, "mm_qin_fold: K %d needs %d pieces a lane (at most 4)", K, L);
+    // (the kernels hold at most 4 pieces a lane: FOLD_KMAX is 256 pieces, so a team of 64 always does)
+    static_assert(FOLD_KMAX / 32 <= 64 * 4, "a row's pieces fit a team of 64 lanes");
+    pick_team(a.P, &a.T, Lp, nullptr, 4);
     *ap = a;
-    *Lp = L;
     return OTPU_OK;
 }
 }  // namespace otpu

@@ -1,0 +1,66 @@
+"""`mxu.dot` itself at the edges of the rules that pick its launches, against the C oracle's MM a range
+(`opentpu/compiler.py:2686-2720`) bit for bit."""
+import numpy as np
+import pytest
+
+from conftest import same_bits
+from oracle import chain as CH
+from oracle import cpu as OC
+from oracle import formats as Q
+from oracle import fp32 as F
+from test_gpu_gemm4 import say, spread
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.fixture(scope="module")
+def mxu():
+    import torch
+    assert torch.cuda.is_available(), "GPU tests need a GPU"
+    from opentpu_amd import _lib, mxu
+    _lib.load()
+    return mxu
+
+
+def packed(rng, N, K, fmt):
+    W = (spread(rng, N, K, 1.5, 128) * 0.02).astype(np.float32)
+    return Q.pack_rsc(W) if fmt == "rsc" else Q.quantize_mxu(W, fmt)
+
+
+def qweight(mxu, rows, srows, fmt, K):
+    return mxu.QWeight.from_packed(rows, srows, "int8" if fmt == "rsc" else fmt, K, fmt == "rsc")
+
+
+@pytest.mark.parametrize("fmt", ["int4", "fp4", "nvfp4"])
+def test_one_row_in_ranges_of_every_width(mxu, fmt):
+    """One row, 4-bit weights: K every multiple of 256 up to 8192, in ranges of 256 and of half of K or
+    K's chunk (`opentpu/kernels/mlp.py:8-30`)."""
+    from opentpu_amd.chain import down_chunk
+    rng = np.random.default_rng(11)
+    N = 40
+    rows, srows = packed(rng, N, 8192, fmt)
+    x = spread(rng, 1, 8192, 2.0, 32)
+    for K in range(512, 8192 + 1, 256):
+        r = np.ascontiguousarray(rows[:, :K // 2])
+        w = qweight(mxu, r, srows, fmt, K)
+        for width in sorted({256, down_chunk(K, fmt), K // 2 if K % 512 == 0 else K}):
+            say("one row", fmt, K, width)
+            got = mxu.dot(np.ascontiguousarray(x[:, :K]), w, ranges=[width] * (K // width))
+            assert same_bits(got, CH.ranges_dot(x[:, :K], (r, srows), fmt, width, mm=OC.mm)), (K, width)
+
+
+@pytest.mark.parametrize("fmt,F_dim", [("int4", 2304), ("nvfp4", 2560), ("fp4", 4864)])
+def test_chain_of_widths_the_fold_splits_evenly(mxu, fmt, F_dim):
+    """A chain whose down projection has 72, 80 or 152 pieces a row: the persistent step and the launches
+    a linear."""
+    from opentpu_amd.chain import DecodeChain, Shape
+    sh = Shape(hidden=256, q_dim=512, kv_dim=256, F=F_dim, layers=2)
+    say("chain", fmt, F_dim)
+    ch = DecodeChain.synthetic(sh, fmt, seed0=41, std=0.05)
+    host = [{k: (r.cpu().numpy(), s.cpu().numpy()) for k, (r, s) in l.items()} for l in ch.layers]
+    x = np.random.default_rng(5).standard_normal((1, 256)).astype(np.float32)
+    want = CH.step(x, host, fmt, 512, F_dim, None, mm=OC.mm)
+    assert ch.persistent and same_bits(ch.step(x).cpu().numpy(), want)
+    assert ch.chain_error() == 0
+    ch.persistent = False
+    assert same_bits(ch.step(x).cpu().numpy(), want)
