@@ -322,8 +322,14 @@ extern "C" int otpu_mm_dot(const int8_t* q, int64_t ldq, const float* Sa, const 
         return otpu_fail(OTPU_EINVAL, "mm_dot: ranges of %d over K %d (multiples of %d for this format)", width, K, chunk);
     if (flags & OTPU_RMAX) return otpu_fail(OTPU_EINVAL, "mm_dot: no RMAX");
     if (act < OTPU_ACT_ANY || act > OTPU_ACT_MX) return otpu_fail(OTPU_EINVAL, "mm_dot: act %d", act);
-    int rc = check_mm("mm_dot", q, ldq, da, ldda, M, K, w, rs, ws, srs, N, fmt, flags, k0);
+    // each range is an MM of its own (the last one's blocks the furthest); the strides hold the whole row
+    const bool plain = (flags & (OTPU_UNIT | OTPU_RSC)) != 0;
+    int rc = check_mm("mm_dot", q, ldq, da, ldda, M, width, w, rs, ws, srs, N, fmt, flags,
+                      plain || k0 < 0 ? k0 : k0 + (K - width) / OTPU_D);
     if (rc) return rc;
+    if (ldq < K || ldda < K / 32 || rs < (fmt == OTPU_INT8 ? K : K / 2))
+        return otpu_fail(OTPU_EINVAL, "mm_dot: ldq %lld, ldda %lld, rs %lld short of K %d", (long long)ldq, (long long)ldda,
+                         (long long)rs, K);
     if (!Sa || !out || ors < N) return otpu_fail(OTPU_EINVAL, "mm_dot: Sa / out NULL or ors < N");
     if ((flags & OTPU_ASCALE) && !alpha) return otpu_fail(OTPU_EINVAL, "mm_dot: ASCALE without alpha");
     hipStream_t s = (hipStream_t)stream;
@@ -334,7 +340,8 @@ extern "C" int otpu_mm_dot(const int8_t* q, int64_t ldq, const float* Sa, const 
         return launch_gemv(a, fmt, 1, s);
     }
     rc = mm_rows(q, ldq, Sa, da, ldda, M, K, R, w, rs, ws, srs, N, fmt, flags & ~OTPU_PAIR, k0, act, alpha, out, ors, s);
-    return rc > 0 ? otpu_fail(OTPU_EALIGN, "mm_dot: offset rows of whole words (da, ldda multiples of 4)") : rc;
+    return rc > 0 ? otpu_fail(OTPU_EALIGN, "mm_dot: offset rows of whole words (da, ldda multiples of 4), ldq below 16 MiB")
+                  : rc;
 }
 
 namespace otpu {

@@ -199,6 +199,7 @@ def C_ptr(t, off: int):
 QIN_ROWS = 16384
 QIN_COLS = 16384                                          # columns otpu_mm_qin's prologue holds
 FOLD_COLS = 8192                                          # ... and otpu_mm_qin_fold's
+OFF_COLS = 1 << 24                                        # otpu_mm_dot's rows: 32-bit offsets over a tile's rows
 
 
 def _dot_row(x, w: QWeight, ranges, out) -> bool:
@@ -272,7 +273,7 @@ def dot(x, w: QWeight, acc=None, out=None, ranges=None, row_mode: bool = False, 
     unit = w.srows is None
     chunk = D if w.fmt == "int8" else 2 * D
     width = ranges[0]
-    one = not rowmax and (len(ranges) == 1 or (min(ranges) == max(ranges) and width % chunk == 0))
+    one = not rowmax and K < OFF_COLS and (len(ranges) == 1 or (min(ranges) == max(ranges) and width % chunk == 0))
     if operand and one:                                   # scales of other strides, offsets of odd addresses: a launch a range
         one = da.data_ptr() % 4 == 0 and (len(ranges) == 1 or (
             isinstance(Sa, X.torch().Tensor) and Sa.is_contiguous() and Sa.shape[1] == M))

@@ -34,3 +34,29 @@ def test_fold_takes_every_row(fmt):
                            None) is None, K
     rs, srs = row_bytes(fmt, 8448)
     assert refusal("otpu_mm_qin_fold", P, None, None, None, 8448, 256, P, rs, P, srs, 8, X.FMT[fmt], 0, 0, P, None)
+
+
+def dot_refusal(fmt, M, K, width, *, ldq=None, ldda=None, rs=None, srs=None, k0=0, flags=0):
+    r, sr = row_bytes(fmt, K + 128 * k0)
+    return refusal("otpu_mm_dot", P, K if ldq is None else ldq, P, P, K // 32 if ldda is None else ldda, M, K, width, P,
+                   r if rs is None else rs, P, sr if srs is None else srs, 8, X.FMT[fmt], flags, k0, 0, None, P, 8, None)
+
+
+@pytest.mark.parametrize("fmt", ["int8", "int4", "nvfp4"])
+def test_mm_dot_checks_a_range(fmt):
+    """otpu_mm_dot over more columns than one MM takes: a range's columns are checked, the strides and the
+    last range's scale blocks against the whole row."""
+    K = 40960
+    r, sr = row_bytes(fmt, K)
+    for M in (1, 8, 300):
+        assert dot_refusal(fmt, M, K, 5120) is None
+        assert dot_refusal(fmt, M, K, 5120, k0=2) is None
+        assert "at most" in dot_refusal(fmt, M, K, K)
+        assert dot_refusal(fmt, M, K, 5120, ldq=K - 16)
+        assert dot_refusal(fmt, M, K, 5120, ldda=K // 32 - 4)
+        assert dot_refusal(fmt, M, K, 5120, rs=r - 16)
+        assert dot_refusal(fmt, M, K, 5120, srs=sr - 16)
+        assert dot_refusal(fmt, M, K, 5120, k0=-1)
+        assert dot_refusal(fmt, M, K, 5120, srs=8 if fmt != "nvfp4" else 16)
+        if fmt != "nvfp4":                                # (plain rows: a scale a row, no blocks)
+            assert dot_refusal(fmt, M, K, 5120, srs=8, flags=X.RSC) is None

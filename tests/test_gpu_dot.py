@@ -7,7 +7,7 @@ from conftest import same_bits
 from oracle import chain as CH
 from oracle import cpu as OC
 from oracle import formats as Q
-from oracle import fp32 as F
+from oracle import mm as MM
 from test_gpu_gemm4 import say, spread
 
 pytestmark = pytest.mark.gpu
@@ -64,3 +64,29 @@ def test_chain_of_widths_the_fold_splits_evenly(mxu, fmt, F_dim):
     assert ch.chain_error() == 0
     ch.persistent = False
     assert same_bits(ch.step(x).cpu().numpy(), want)
+
+
+@pytest.mark.parametrize("fmt,M,K,width", [("int8", 8, 40960, 5120), ("int4", 1, 40960, 5120), ("nvfp4", 3, 33024, 768),
+                                           ("rsc", 40, 32768, 16384), ("int4", 1, 1 << 24, 16384)])
+def test_ranges_past_one_mms_columns(mxu, fmt, M, K, width):
+    """More columns than one MM takes (32640), each range within; and past 32-bit offsets in a tile."""
+    import torch
+    rng = np.random.default_rng(K + M)
+    N = 9 if K < 1 << 20 else 2
+    base, sr = packed(rng, N, width, fmt)
+    R = K // width
+    rows = np.concatenate([np.roll(base, i % N, 0) for i in range(R)], 1)
+    head = {"nvfp4": 16, "int4": 8}.get(fmt, 4)
+    per = {"int8": 1, "int4": 4, "nvfp4": 8, "rsc": 0}[fmt] * width // 128
+    srows = np.concatenate([sr[:, :head]] + [np.roll(sr[:, head:head + per], i % N, 0) for i in range(R)], 1)
+    x = rng.standard_normal((M, K)).astype(np.float32)
+    say("ranges past one MM", fmt, M, K, width)
+    got = mxu.dot(torch.from_numpy(x).cuda(), qweight(mxu, rows, srows, fmt, K), ranges=[width] * R).cpu().numpy()
+    want = None
+    for r in range(R):
+        q, Sa, da = OC.qact(x[:, r * width:(r + 1) * width])
+        b = base.shape[1]
+        want = OC.mm(q, Sa, da, np.ascontiguousarray(rows[:, r * b:(r + 1) * b]), srows, "int8" if fmt == "rsc" else fmt,
+                     width, flags=(MM.RSC if fmt == "rsc" else 0) | (MM.ACC if r else 0),
+                     k0=0 if fmt == "rsc" else r * width // 128, old=want)
+    assert same_bits(got, want)
