@@ -159,8 +159,9 @@ int otpu_mm_dot(const int8_t* q, int64_t ldq, const float* Sa, const uint8_t* da
  * nsum - 1 more rows sum_stride apart in order (x_0 + x_1 + ..: the ACC chain of a previous
  * per-range MM, opentpu/isasim.py:899-905), times xmul when given (VOP MUL), then QACT's
  * RSCALE and CSCALE products (x * rscale[0]) * cscale[c] when given (rscale: one float, the
- * row's factor; cscale [K]; docs/isa.md:447-452).  No ACC / ASCALE / RMAX; width at most 4096,
- * a multiple of 128 (int8) or 256 (4-bit); nsum at most 16. */
+ * row's factor; cscale [K]; docs/isa.md:447-452).  No ACC / ASCALE / RMAX; width at most 16384,
+ * a multiple of 128 (int8) or 256 (4-bit); nsum at most 16.  out must not overlap x, xmul, rscale or
+ * cscale: every workgroup reads them while others store. */
 int otpu_mm_qin(const float* x, const float* xmul, const float* rscale, const float* cscale, int nsum,
                 int64_t sum_stride, int K, int width, const uint8_t* w, int64_t rs, const uint8_t* ws,
                 int64_t srs, int N, int fmt, int flags, int k0, float* out, int64_t ors, int64_t part_stride,
@@ -174,7 +175,7 @@ int otpu_mm_qin(const float* x, const float* xmul, const float* rscale, const fl
  * own QACT and multiplied by its weight columns, and the ranges' outputs added in range order into
  * out[0..N): otpu_mm_qin's ranges and the fold of their rows, bit for bit.  4-bit weights with
  * scale rows only (INT4, FP4, NVFP4; no flags but PAIR); K a multiple of 256, at most 8192; width
- * a multiple of 256 that divides K. */
+ * a multiple of 256 that divides K.  out must not overlap x, xmul, rscale or cscale (as otpu_mm_qin). */
 int otpu_mm_qin_fold(const float* x, const float* xmul, const float* rscale, const float* cscale, int K,
                      int width, const uint8_t* w, int64_t rs, const uint8_t* ws, int64_t srs, int N, int fmt,
                      int flags, int k0, float* out, otpu_stream_t stream);

@@ -202,11 +202,18 @@ FOLD_COLS = 8192                                          # ... and otpu_mm_qin_
 OFF_COLS = 1 << 24                                        # otpu_mm_dot's rows: 32-bit offsets over a tile's rows
 
 
+def _overlap(a, b) -> bool:
+    """Whether the memory two contiguous tensors hold overlaps."""
+    pa, pb = a.data_ptr(), b.data_ptr()
+    return pa < pb + b.numel() * b.element_size() and pb < pa + a.numel() * a.element_size()
+
+
 def _dot_row(x, w: QWeight, ranges, out) -> bool:
     """One fp32 row x (a contiguous device tensor [1, K]) @ w^T into out in one launch, QACT and the
-    ranges' ACC chain inside; False where no such kernel takes the call."""
+    ranges' ACC chain inside; False where no such kernel takes the call, or out overlaps x (every
+    workgroup reads the row while others store)."""
     K, chunk = w.K, (D if w.fmt == "int8" else 2 * D)
-    if w.N > QIN_ROWS or x.data_ptr() % 16 or K % chunk:
+    if w.N > QIN_ROWS or x.data_ptr() % 16 or K % chunk or _overlap(x, out):
         return False
     ws, srs = (0, 0) if w.srows is None else (w.srows.data_ptr(), w.srows.shape[1])
     fl = _flags(w.srows is None, w.rsc)

@@ -90,3 +90,21 @@ def test_ranges_past_one_mms_columns(mxu, fmt, M, K, width):
                      width, flags=(MM.RSC if fmt == "rsc" else 0) | (MM.ACC if r else 0),
                      k0=0 if fmt == "rsc" else r * width // 128, old=want)
     assert same_bits(got, want)
+
+
+@pytest.mark.parametrize("fmt,K,width", [("int8", 1024, 1024), ("int4", 4096, 4096), ("nvfp4", 2048, 256), ("int8", 1024, 256)])
+def test_one_row_written_over(mxu, fmt, K, width):
+    """out= on the row that is multiplied, or on a part of it."""
+    import torch
+    rng = np.random.default_rng(K + width)
+    rows, srows = packed(rng, K, K, fmt)
+    w = qweight(mxu, rows, srows, fmt, K)
+    x = spread(rng, 1, K, 2.0, 32)
+    want = CH.ranges_dot(x, (rows, srows), fmt, width, mm=OC.mm)
+    say("one row written over", fmt, K, width)
+    for off in (0, 4, -8, K // 2):
+        buf = torch.zeros((3 * K,), device="cuda")
+        xd, out = buf[K:2 * K].view(1, K), buf[K + off:2 * K + off].view(1, K)
+        xd.copy_(torch.from_numpy(x))
+        assert mxu.dot(xd, w, out=out, ranges=[width] * (K // width)) is out
+        assert same_bits(out.cpu().numpy(), want), off
