@@ -281,9 +281,10 @@ def dot(x, w: QWeight, acc=None, out=None, ranges=None, row_mode: bool = False, 
     chunk = D if w.fmt == "int8" else 2 * D
     width = ranges[0]
     one = not rowmax and K < OFF_COLS and (len(ranges) == 1 or (min(ranges) == max(ranges) and width % chunk == 0))
-    if operand and one:                                   # scales of other strides, offsets of odd addresses: a launch a range
-        one = da.data_ptr() % 4 == 0 and (len(ranges) == 1 or (
-            isinstance(Sa, X.torch().Tensor) and Sa.is_contiguous() and Sa.shape[1] == M))
+    if operand and one:                                   # ranges short of the row, scales of other shapes or
+        one = (da.data_ptr() % 4 == 0 and sum(ranges) == K  # strides, offsets of odd addresses: a launch a range
+               and (len(ranges) == 1 or (isinstance(Sa, X.torch().Tensor) and Sa.is_contiguous()
+                                         and Sa.dim() == 2 and Sa.shape[0] >= len(ranges) and Sa.shape[1] == M)))
     if not operand and not one:
         q, Sa, da, ranges = quantize_ranges(xd, ranges, row_mode)
     y = X.dev(acc, np.float32) if acc is not None else (out if out is not None else X.empty((M, N), np.float32))

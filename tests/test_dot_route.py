@@ -38,3 +38,30 @@ def test_a_row_written_over_is_quantized_first(calls, fmt, ranges):
         mxu.dot(x, w, out=buf[o0:o0 + N].view(1, N), ranges=ranges)
         names = [c[0] for c in calls]
         assert names[0].startswith("otpu_qact" if over else "otpu_mm_qin"), (o0, names)
+
+
+def operand(M, K, ranges, sa_rows=None):
+    R = len(ranges) if sa_rows is None else sa_rows
+    return torch.zeros((M, K), dtype=torch.int8), torch.zeros((R, M)), torch.zeros((M, K // 32), dtype=torch.uint8), ranges
+
+
+@pytest.mark.parametrize("M", [1, 6])
+def test_an_operand_is_read_no_further_than_it_goes(calls, M):
+    """Ranges over a part of the operand's columns, and scales that are not a row a range, run a launch a
+    range: otpu_mm_dot takes its ranges from K, and a scale a range and row."""
+    w = weight(64, 1024, "int4")
+    for ranges in ([256], [256, 256], [512]):
+        calls.clear()
+        mxu.dot(operand(M, 1024, ranges), w)
+        assert [c[0] for c in calls] == ["otpu_mm"] * len(ranges), ranges
+        assert [c[7] for c in calls] == ranges
+    q, Sa, da, rg = operand(M, 1024, [256] * 4)
+    for S in (list(Sa), Sa.t().contiguous().t(), Sa.repeat(1, 2)[:, :M]) + ((Sa[:, 0],) if M == 1 else ()):
+        calls.clear()
+        mxu.dot((q, S, da, rg), w)
+        want = ["otpu_mm_dot"] if isinstance(S, torch.Tensor) and S.dim() == 2 and S.is_contiguous() else ["otpu_mm"] * 4
+        assert [c[0] for c in calls] == want
+    calls.clear()
+    with pytest.raises(IndexError):
+        mxu.dot(operand(M, 1024, [256] * 4, sa_rows=3), w)
+    assert "otpu_mm_dot" not in [c[0] for c in calls]

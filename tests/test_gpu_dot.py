@@ -108,3 +108,21 @@ def test_one_row_written_over(mxu, fmt, K, width):
         xd.copy_(torch.from_numpy(x))
         assert mxu.dot(xd, w, out=out, ranges=[width] * (K // width)) is out
         assert same_bits(out.cpu().numpy(), want), off
+
+
+@pytest.mark.parametrize("fmt,M", [("int8", 7), ("int4", 1), ("fp4", 70)])
+def test_ranges_over_a_part_of_an_operand(mxu, fmt, M):
+    """An operand's ranges may cover its first columns only; a scale a range as a vector (one row)."""
+    import torch
+    rng = np.random.default_rng(M)
+    N, K = 50, 1024
+    rows, srows = packed(rng, N, K, fmt)
+    w = qweight(mxu, rows, srows, fmt, K)
+    x = torch.from_numpy(spread(rng, M, K, 2.0, 32)).cuda()
+    q, Sa, da, _ = mxu.quantize_ranges(x, [256] * 4)
+    host = x.cpu().numpy()
+    for R in (1, 2, 4):
+        say("ranges over a part", fmt, M, R)
+        want = CH.ranges_dot(host[:, :256 * R], (rows, srows), fmt, 256, mm=OC.mm)
+        for S in (Sa[:R],) + ((Sa[:R, 0].contiguous(),) if M == 1 else ()):
+            assert same_bits(mxu.dot((q, S, da, [256] * R), w).cpu().numpy(), want)
