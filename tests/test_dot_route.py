@@ -65,3 +65,10 @@ def test_an_operand_is_read_no_further_than_it_goes(calls, M):
     with pytest.raises(IndexError):
         mxu.dot(operand(M, 1024, [256] * 4, sa_rows=3), w)
     assert "otpu_mm_dot" not in [c[0] for c in calls]
+
+
+@pytest.mark.parametrize("shape", [(1024,), (1, 1024, 1024), (2, 1024, 3)])
+def test_rows_are_a_matrix(calls, shape):
+    with pytest.raises(ValueError):
+        mxu.dot(torch.zeros(shape), weight(64, 1024, "int4"))
+    assert not calls
