@@ -264,13 +264,11 @@ def dot(x, w: QWeight, acc=None, out=None, ranges=None, row_mode: bool = False, 
         M, K = xd.shape
         if K != w.K:
             raise ValueError(f"dot: K mismatch {K} vs {w.K}")
-        if M == 1 and not (row_mode or rowmax) and acc is None and acc_scale is None:
-            rl = [K] if ranges is None else list(ranges)
-            if sum(rl) == K and not any(r % D for r in rl):
-                y = out if out is not None else X.empty((1, N), np.float32)
-                if _dot_row(xd, w, rl, y):
-                    return X.host(y) if numpy_in else y
         ranges = _check_ranges(ranges, K)
+        if M == 1 and not (row_mode or rowmax) and acc is None and acc_scale is None:
+            y = out if out is not None else X.empty((1, N), np.float32)
+            if _dot_row(xd, w, ranges, y):
+                return X.host(y) if numpy_in else y
     else:
         q, Sa, da, ranges = x
         M, K = q.shape

@@ -72,3 +72,14 @@ def test_rows_are_a_matrix(calls, shape):
     with pytest.raises(ValueError):
         mxu.dot(torch.zeros(shape), weight(64, 1024, "int4"))
     assert not calls
+
+
+@pytest.mark.parametrize("M,fmt,widths", [(1, "int8", [256] * 4), (1, "int4", [512, 256, 256]), (3, "int4", [256] * 4)])
+def test_ranges_are_read_once(calls, M, fmt, widths):
+    """Any iterable of widths, as a list of them."""
+    made = []
+    for ranges in (widths, tuple(widths), iter(widths)):
+        calls.clear()
+        mxu.dot(torch.zeros((M, 1024)), weight(64, 1024, fmt), ranges=ranges)
+        made.append([c[0] for c in calls])
+    assert made[0] == made[1] == made[2] and made[0]
