@@ -26,10 +26,10 @@ typedef int v4i __attribute__((ext_vector_type(4)));
 
 // The windows of a block's int32 sums: activation offsets up to D and (by dw <= W - D) no dropped
 // term.  Bounds of a block's |t| = sum over 4 groups of |c m| 2^D, all below 2^31:
-//   int8:  |c| <= 32 127 127, D 8:               2^19 2^8 4                  = 5.3e8
-//   int4:  the MFMA multiplies 16 w: 16 32 127 8 63, D 4:                    = 2.1e9
-//   fp4:   |w| <= 12: 32 127 12 63 4, D 6:                                   = 7.9e8
-//   nvfp4: two 16-groups, m 2^(E - Eb + 3) <= 15 8: 16 127 12 120 8, D 6:    = 1.5e9
+//   int8:  |c| <= 32 128 128, D 8:               2^19 2^8 4                  = 5.4e8
+//   int4:  the MFMA multiplies 16 w: 16 32 128 8 63 4, D 4:                  = 2.114e9
+//   fp4:   |w| <= 12: 32 128 12 63 4, D 6:                                   = 7.9e8
+//   nvfp4: two 16-groups, m 2^(E - Eb + 3) <= 15 8: 16 128 12 120 8, D 6:    = 1.51e9
 // A block with an offset outside them takes the group-by-group double path (exact for any).
 template <int FMT>
 struct Win {

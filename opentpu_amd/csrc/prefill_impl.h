@@ -39,14 +39,15 @@ typedef short s2 __attribute__((ext_vector_type(2)));
 
 constexpr int TN = 128;                     // weight rows a workgroup
 
-// |sum of one block| <= BB 2^(ew + sd) in the wave's units (4 groups of 32 terms):
-//   int8 32 127 127 4; int4 32 127 8 63 4; fp4 32 127 12 63 4; nvfp4 16 127 12 15 8
+// |sum of one block| <= BB 2^(ew + sd) in the wave's units (4 groups of 32 terms; any int8 activation,
+// -128 too, which QACT never gives):
+//   int8 32 128 128 4; int4 32 128 8 63 4; fp4 32 128 12 63 4; nvfp4 16 128 12 15 8
 template <int FMT>
 struct Win {
     static constexpr int W = FMT == OTPU_INT8 ? 16 : (FMT == OTPU_NVFP4 ? 13 : 11);
-    static constexpr int64_t BB = FMT == OTPU_INT8 ? 32 * 127 * 127 * 4
-                                : FMT == OTPU_INT4 ? 32 * 127 * 8 * 63 * 4
-                                : FMT == OTPU_FP4  ? 32 * 127 * 12 * 63 * 4 : 16 * 127 * 12 * 15 * 8;
+    static constexpr int64_t BB = FMT == OTPU_INT8 ? 32 * 128 * 128 * 4
+                                : FMT == OTPU_INT4 ? 32 * 128 * 8 * 63 * 4
+                                : FMT == OTPU_FP4  ? 32 * 128 * 12 * 63 * 4 : 16 * 128 * 12 * 15 * 8;
     static constexpr int SMAX = FMT == OTPU_INT8 ? 9 : (FMT == OTPU_NVFP4 ? 9 : 7);
     static_assert((BB << SMAX) + 65536 < (1ll << 31), "a block's sum fits int32");
     static_assert(SMAX <= W, "no term of the windows is dropped");

@@ -104,6 +104,35 @@ def test_prefill_largest_products(X, fmt, lo, hi):
     assert same_bits(got[:, :40], OC.mm(q, Sa, da, cut(rows[:40]), cut(srows[:40]), fmt, K))
 
 
+@pytest.mark.parametrize("fmt,K,sd,M,N", [("int8", 256, 9, 100, 8100), ("int8", 512, 8, 520, 8200), ("int4", 16768, 1, 100, 8100),
+                                          ("fp4", 11136, 1, 100, 8100), ("nvfp4", 23424, 2, 100, 8100)])
+def test_prefill_sums_of_lowest_values(X, fmt, K, sd, M, N):
+    """Activations of -128 on the largest weights and multipliers, one row at offset 0 beside rows at
+    sd: the block sums a count of 127 a value would let past 2^31 (int8 2 * 4 * 32 * 128 * 128 * 2^9)."""
+    KB = K // 128
+    byte = {"int8": 0x80, "int4": 0x88, "fp4": 0xFF, "nvfp4": 0xFF}[fmt]
+    rows = np.full((N, KB * (128 if fmt == "int8" else 64)), byte, np.uint8)
+    one = np.ones((N, 1), np.float32).view(np.uint8)
+    if fmt == "int8":
+        srows = one
+    elif fmt == "nvfp4":                                  # E 15, m 15: the largest multiplier, offset 0
+        srows = np.concatenate([one, np.zeros((N, 12), np.uint8), np.full((N, 8 * KB + 8 * (KB & 1)), 0x7F, np.uint8)], 1)
+    else:
+        word = np.full((N, KB + (KB & 1)), sum(63 << (8 + 6 * b) for b in range(4)), np.uint32)
+        srows = np.concatenate([one, np.zeros((N, 4), np.uint8), word.view(np.uint8).reshape(N, -1)], 1)
+    q = np.full((M, K), -128, np.int8)
+    q[3::5] = 127
+    da = np.full((M, K // 32), sd, np.uint8)
+    da[::7] = 0
+    Sa = np.ones(M, np.float32)
+    fl = MM.RSC if fmt == "int8" else 0
+    say("prefill lowest values", fmt, K)
+    got = mm_dot(X, q, Sa, da, rows, srows, fmt, K, K, fl, act=2)
+    cut = np.ascontiguousarray
+    assert same_bits(got[:, :40], OC.mm(q, Sa, da, cut(rows[:40]), cut(srows[:40]), fmt, K, flags=fl))
+    assert same_bits(got[:, N - 8:], OC.mm(q, Sa, da, cut(rows[N - 8:]), cut(srows[N - 8:]), fmt, K, flags=fl))
+
+
 @pytest.mark.parametrize("fmt", ["int8", "int4", "nvfp4"])
 def test_prefill_long_sums(X, fmt):
     """Sums that leave int32 inside the walk: every product at its largest over K = 16384."""
