@@ -5,7 +5,7 @@
 // negative).  A tile whose groups all carry one offset d is a plain int8 GEMM.  With two offsets the
 // sum splits into two planes of masked activations, C_0 and C_1, each an int32 matrix product:
 //     acc = 2^(16 - smax) * sum_p 2^(smax - d_p) * C_p,
-// within int32 where K * 127^2 * 2^(smax - dmin) stays below 2^31 (checked per tile).  A tile of
+// within int32 where K * 128^2 * 2^(smax - dmin) stays below 2^31 (checked per tile).  A tile of
 // more offsets takes prefill_impl.h's walk, which adds each group's products with its own shift (the
 // masked operand planes it had taken one K walk each: c3's shape with activations of three offsets
 // 67 us).
@@ -545,8 +545,8 @@ __global__ __launch_bounds__(512) void gemm_lw_kernel(GemmArgs a) {
     const bool over = (dall >> 17) & 1;
     const int np = __builtin_popcount(dmask);
     const int dmin = dmask ? __builtin_ctz(dmask) : 0, smax = dmask ? 31 - __builtin_clz(dmask) : 0;
-    // the planes' sum in int32: |acc| <= K 127^2 2^(smax - dmin)
-    const bool fits = (int64_t)a.K * 16129 <= (((int64_t)1 << 31) - 1) >> (smax - dmin);
+    // the planes' sum in int32: |acc| <= K 128^2 2^(smax - dmin)
+    const bool fits = (int64_t)a.K * 16384 <= (((int64_t)1 << 31) - 1) >> (smax - dmin);
     const bool single = np == 1 && !over;
 
     // a full tile's epilogue is shared: waves 0-3 write their transposes, then wave w and its

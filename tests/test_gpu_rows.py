@@ -133,6 +133,24 @@ def test_prefill_sums_of_lowest_values(X, fmt, K, sd, M, N):
     assert same_bits(got[:, N - 8:], OC.mm(q, Sa, da, cut(rows[N - 8:]), cut(srows[N - 8:]), fmt, K, flags=fl))
 
 
+@pytest.mark.parametrize("K,top", [(2048, 6), (4096, 5), (1024, 7), (2048, 5)])
+def test_gemm_sums_of_lowest_values(X, K, top):
+    """The int8 GEMM's two planes (offsets 0 and top a tile) of -128s: K 128^2 2^top reaches 2^31 (the last
+    case half of it: the planes take it)."""
+    M, N = 512, 8192
+    rows = np.full((N, K), 0x80, np.uint8)
+    rows[1::2] = 0x7F
+    srows = np.ones((N, 1), np.float32).view(np.uint8)
+    q = np.full((M, K), -128, np.int8)
+    da = np.zeros((M, K // 32), np.uint8)
+    da[5::64] = top
+    Sa = np.ones(M, np.float32)
+    say("gemm lowest values", K, top)
+    got = mm_dot(X, q, Sa, da, rows, srows, "int8", K, K, MM.RSC, act=0)
+    cut = np.ascontiguousarray
+    assert same_bits(got[:, 1000:1020], OC.mm(q, Sa, da, cut(rows[1000:1020]), cut(srows[1000:1020]), "int8", K, flags=MM.RSC))
+
+
 @pytest.mark.parametrize("fmt", ["int8", "int4", "nvfp4"])
 def test_prefill_long_sums(X, fmt):
     """Sums that leave int32 inside the walk: every product at its largest over K = 16384."""
