@@ -24,19 +24,20 @@ int otpu_batch_try(const int8_t* q, int64_t ldq, const float* Sa, const uint8_t*
     // int4 41): us at 64 -> at 32, QACT in: int8 512 x 2048 x 1024 22.1 -> 18.3, 512 x 3072 x 1024 in ranges of 256
     // 46.0 -> 31.9, 100 x 2048 x 6000 36.3 -> 29.1; nvfp4 29.6 -> 26.0, 61.7 -> 46.7, 49.9 -> 43.2; fp4's ranges 40.2
     // -> 37.4, int4's 37.6 -> 36.4, but without ranges int4 100 x 2048 x 6000 31.7 -> 33.4, fp4 34.7 -> 34.8
-    const bool spills = fmt == OTPU_INT8 || fmt == OTPU_NVFP4 || ranges > 1;
-    int nsub = mt == 2 && spills ? 2 : 4;
+    int nsub = mt == 2 && (!bt::has_wide_tile(fmt) || ranges > 1) ? 2 : 4;
     while (nsub > 1 && (int64_t)((N + 16 * nsub - 1) / (16 * nsub)) * tiles_m * kwmax < want) nsub >>= 1;
     int kw = 1;
     while (kw < kwmax && (int64_t)((N + 16 * nsub - 1) / (16 * nsub)) * tiles_m * kw < want) kw <<= 1;
     a.kw = kw;
     a.tiles_n = (N + 16 * nsub - 1) / (16 * nsub);
     a.groups_m = (int)(((M + 16 * mt - 1) / (16 * mt) + 8 / kw - 1) / (8 / kw));
+    bool ok;
     switch (fmt) {
-        case OTPU_INT8: bt::launch_fmt<OTPU_INT8>(a, nsub, mt, s); break;
-        case OTPU_INT4: bt::launch_fmt<OTPU_INT4>(a, nsub, mt, s); break;
-        case OTPU_FP4: bt::launch_fmt<OTPU_FP4>(a, nsub, mt, s); break;
-        default: bt::launch_fmt<OTPU_NVFP4>(a, nsub, mt, s); break;
+        case OTPU_INT8: ok = bt::launch_fmt<OTPU_INT8>(a, nsub, mt, s); break;
+        case OTPU_INT4: ok = bt::launch_fmt<OTPU_INT4>(a, nsub, mt, s); break;
+        case OTPU_FP4: ok = bt::launch_fmt<OTPU_FP4>(a, nsub, mt, s); break;
+        default: ok = bt::launch_fmt<OTPU_NVFP4>(a, nsub, mt, s); break;
     }
+    if (!ok) return otpu_fail(OTPU_EINVAL, "mm batch: no kernel of format %d for %d x %d rows a wave", fmt, 16 * nsub, 16 * mt);
     return otpu_launch_check("mm batch");
 }

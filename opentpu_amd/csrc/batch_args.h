@@ -21,8 +21,13 @@ struct Args {
     int tiles_n, groups_m;          // tiles of 16 NSUB weight rows; groups of 8 / kw row tiles
 };
 
+// the formats with a kernel of 64 weight rows beside 32 activation rows a wave (nsub 4, mt 2); in the others 32
+// weight rows are the faster (batch.hip's rule)
+constexpr bool has_wide_tile(int fmt) { return fmt == OTPU_INT4 || fmt == OTPU_FP4; }
+
+// false: no such kernel (nothing launched)
 template <int FMT>
-void launch_fmt(const Args& a, int nsub, int mt, hipStream_t s);
+bool launch_fmt(const Args& a, int nsub, int mt, hipStream_t s);
 
 }  // namespace bt
 }  // namespace otpu

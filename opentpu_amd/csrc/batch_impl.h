@@ -432,16 +432,23 @@ static void launch(const Args& a, hipStream_t s) {
 }
 
 template <int FMT>
-void launch_fmt(const Args& a, int nsub, int mt, hipStream_t s) {
+bool launch_fmt(const Args& a, int nsub, int mt, hipStream_t s) {
     if (mt == 1) {
         if (nsub == 1) launch<FMT, 1, 1>(a, s);
         else if (nsub == 2) launch<FMT, 2, 1>(a, s);
         else launch<FMT, 4, 1>(a, s);
-    } else {
-        if (nsub == 1) launch<FMT, 1, 2>(a, s);
-        else if (nsub == 2) launch<FMT, 2, 2>(a, s);
-        else if constexpr (FMT == OTPU_INT4 || FMT == OTPU_FP4) launch<FMT, 4, 2>(a, s);   // (others: batch.hip's rule)
+        return true;
     }
+    if (nsub == 1) {
+        launch<FMT, 1, 2>(a, s);
+        return true;
+    }
+    if (nsub == 2) {
+        launch<FMT, 2, 2>(a, s);
+        return true;
+    }
+    if constexpr (has_wide_tile(FMT)) launch<FMT, 4, 2>(a, s);
+    return has_wide_tile(FMT);
 }
 
 }  // namespace bt

@@ -3,6 +3,6 @@
 
 namespace otpu {
 namespace bt {
-template void launch_fmt<OTPU_INT8>(const Args& a, int nsub, int mt, hipStream_t s);
+template bool launch_fmt<OTPU_INT8>(const Args& a, int nsub, int mt, hipStream_t s);
 }  // namespace bt
 }  // namespace otpu
