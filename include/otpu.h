@@ -180,6 +180,11 @@ int otpu_mm_qin_fold(const float* x, const float* xmul, const float* rscale, con
                      int width, const uint8_t* w, int64_t rs, const uint8_t* ws, int64_t srs, int N, int fmt,
                      int flags, int k0, float* out, otpu_stream_t stream);
 
+/* The columns that all workgroups of an otpu_mm_qin (width K) or otpu_mm_qin_fold (several ranges) launch
+ * quantize together, each the whole row: what one launch costs beside a QACT of its own, for a caller
+ * that has the choice.  0 where the entry point does not take the sizes.  Launches nothing. */
+int64_t otpu_qin_columns(int K, int width, int N, int fmt);
+
 /* MM SPL (split terms: opentpu/isasim.py:757-770, :849-852, :872-873; docs/isa.md:414-441): one
  * MM over a split operand's terms, one K-block (128) of int8 RSC weights a part, natural rows.
  *   q [M, ldq]: the activations' hi part at q[j, 0..128), with nterms 3 also the lo part at

@@ -42,6 +42,7 @@ SIGNATURES = {
     "otpu_mm_dot": ([_P, _L, _P, _P, _L, _I, _I, _I, _P, _L, _P, _L, _I, _I, _I, _I, _I, _P, _P, _L, _P], _I),
     "otpu_vmul": ([_P, _P, _P, _L, _P], _I),
     "otpu_mm_qin": ([_P, _P, _P, _P, _I, _L, _I, _I, _P, _L, _P, _L, _I, _I, _I, _I, _P, _L, _L, _P], _I),
+    "otpu_qin_columns": ([_I, _I, _I, _I], _L),
     "otpu_mm_qin_fold": ([_P, _P, _P, _P, _I, _I, _P, _L, _P, _L, _I, _I, _I, _I, _P, _P], _I),
     "otpu_mm_spl": ([_P, _L, _P, _P, _L, _I, _I, _P, _L, _L, _P, _L, _I, _I, _P, _L, _P], _I),
     "otpu_acc_rows": ([_P, _I, _L, _I, _P, _P, _P], _I),

@@ -447,6 +447,19 @@ extern "C" int otpu_mm_qin_fold(const float* x, const float* xmul, const float* 
     return otpu_launch_check("mm_qin_fold");
 }
 
+extern "C" int64_t otpu_qin_columns(int K, int width, int N, int fmt) {
+    const int chunk = fmt == OTPU_INT8 ? OTPU_D : 2 * OTPU_D;
+    if (fmt < OTPU_INT8 || fmt > OTPU_NVFP4 || N < 1 || width < chunk || width % chunk || K % width) return 0;
+    const bool folded = width < K;
+    if (folded ? fmt == OTPU_INT8 || K > FOLD_KMAX : K > QIN_KBIG) return 0;
+    MMArgs a = {};
+    int L = 1;
+    a.N = N;
+    a.P = (fmt == OTPU_INT8 ? K : K / 2) / 16;
+    pick_team(a.P, &a.T, &L, &a.nseg, folded ? 4 : LMAX);
+    return K * (folded ? fold_blocks(a) : qin_blocks(a, fmt, L, 1));
+}
+
 extern "C" int otpu_acc_rows(const float* parts, int R, int64_t pstride, int n, const float* old, float* out,
                              otpu_stream_t stream) {
     if (!parts || !out || R < 1 || n < 1 || (R > 1 && pstride < n))

@@ -3,6 +3,8 @@
 // each instantiated in its own translation unit (gemv_int8.hip, gemv_int4.hip, gemv_fp4.hip,
 // gemv_nvfp4.hip) so the four compile in parallel.
 #pragma once
+#include <cstdlib>
+
 #include "otpu_common.h"
 
 namespace otpu {
@@ -113,6 +115,48 @@ constexpr bool fits_rt(int fmt, int mr, int L) {
 }
 template <int FMT, int MR, int L>
 constexpr bool fits() { return fits_rt(FMT, MR, L); }
+
+// workgroups per CU the streaming grid aims for (measured on MI355X): for one piece a lane 64,
+// where the 80-problem c2 and the 128-problem c1 give each wave one row group (c2: 7.01-7.03
+// TB/s against 6.58-6.79 at 40, 6.74-6.83 at 32, 6.80-6.82 at 48 and 6.90 at 56, two runs on
+// one box; c1: 6.86-6.92 against 6.59-6.62 at 32); 24 for four or more pieces (the LM head:
+// 103.7-104.4 against 104.6-106.5 us at 16 over four paired runs, 106-108 at 8, 12 or 32),
+// else 8; OTPU_GEMV_BLOCKS_PER_CU overrides
+inline int gemv_blocks_per_cu(int L, int fmt) {
+    (void)fmt;
+    static const int v = [] {                   // read once (thread-safe static initialisation)
+        const char* e = getenv("OTPU_GEMV_BLOCKS_PER_CU");
+        const int x = e ? atoi(e) : 0;
+        return (x > 0 && x <= 64) ? x : 0;
+    }();
+    return v ? v : (L == 1 ? 64 : (L >= 4 ? 24 : 8));
+}
+
+// rows a team takes per iteration (one activation row, one piece a lane) when the default
+// would give fewer workgroups than CUs: a small single GEMV then still spreads over the chip
+constexpr int R_SMALL = 4;
+
+// the grid of a launch with R rows a team: about gemv_blocks_per_cu workgroups per CU over the
+// whole batch, fewer when the rows run out (each wave then streams many row groups; its
+// activation registers are loaded once)
+inline int64_t gemv_blocks(const MMArgs& a, int fmt, int R, int L, int batch) {
+    const int64_t waves = (a.N + (int64_t)R * (64 / a.T) - 1) / ((int64_t)R * (64 / a.T));
+    int64_t blocks = (waves + 3) / 4;
+    int64_t cap = (int64_t)otpu_cu_count() * gemv_blocks_per_cu(L, fmt) / batch;
+    if (cap < 1) cap = 1;
+    return blocks > cap ? cap : blocks;
+}
+
+// the workgroups of one problem of a launch with the QACT of its row in the prologue (launch_qin), and of the
+// folded down projection (launch_fold: a team a row, 4 waves a workgroup, up to 32 workgroups a CU)
+inline int64_t qin_blocks(const MMArgs& a, int fmt, int L, int batch) {
+    const int64_t blocks = gemv_blocks(a, fmt, rows_per_team_rt(L, 1), L, batch);
+    return L == 1 && blocks * batch < otpu_cu_count() ? gemv_blocks(a, fmt, R_SMALL, L, batch) : blocks;
+}
+inline int64_t fold_blocks(const MMArgs& a) {
+    const int64_t rows = 64 / a.T, blocks = ((a.N + rows - 1) / rows + 3) / 4, cap = (int64_t)otpu_cu_count() * 32;
+    return blocks > cap ? cap : blocks;
+}
 
 // launch the streaming GEMV for MR <= 4 activation rows, L pieces a lane (team size a.T)
 template <int FMT>

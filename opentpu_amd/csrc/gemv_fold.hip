@@ -21,13 +21,8 @@ static void launch_fold_fmt(const MMArgs& a, int L, int64_t blocks, hipStream_t 
     }
 }
 
-// the grid: a team a row, 4 waves a workgroup, as many workgroups as rows allow up to 32 a CU
 void launch_fold(const MMArgs& a, int fmt, int L, hipStream_t s) {
-    const int64_t rows_per_wave = 64 / a.T;
-    const int64_t waves = (a.N + rows_per_wave - 1) / rows_per_wave;
-    int64_t blocks = (waves + 3) / 4;
-    const int64_t cap = (int64_t)otpu_cu_count() * 32;
-    if (blocks > cap) blocks = cap;
+    const int64_t blocks = fold_blocks(a);
     if (fmt == OTPU_INT4) launch_fold_fmt<OTPU_INT4>(a, L, blocks, s);
     else if (fmt == OTPU_FP4) launch_fold_fmt<OTPU_FP4>(a, L, blocks, s);
     else launch_fold_fmt<OTPU_NVFP4>(a, L, blocks, s);

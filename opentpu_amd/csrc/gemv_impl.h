@@ -862,37 +862,6 @@ __global__ __launch_bounds__(256) void gemv_qin_kernel(MMArgs a) {
     else gemv_body<FMT, 1, L, 16, PLAIN, true, R>(a);
 }
 
-// workgroups per CU the streaming grid aims for (measured on MI355X): for one piece a lane 64,
-// where the 80-problem c2 and the 128-problem c1 give each wave one row group (c2: 7.01-7.03
-// TB/s against 6.58-6.79 at 40, 6.74-6.83 at 32, 6.80-6.82 at 48 and 6.90 at 56, two runs on
-// one box; c1: 6.86-6.92 against 6.59-6.62 at 32); 24 for four or more pieces (the LM head:
-// 103.7-104.4 against 104.6-106.5 us at 16 over four paired runs, 106-108 at 8, 12 or 32),
-// else 8; OTPU_GEMV_BLOCKS_PER_CU overrides
-inline int gemv_blocks_per_cu(int L, int fmt) {
-    (void)fmt;
-    static const int v = [] {                   // read once (thread-safe static initialisation)
-        const char* e = getenv("OTPU_GEMV_BLOCKS_PER_CU");
-        const int x = e ? atoi(e) : 0;
-        return (x > 0 && x <= 64) ? x : 0;
-    }();
-    return v ? v : (L == 1 ? 64 : (L >= 4 ? 24 : 8));
-}
-
-// rows a team takes per iteration (one activation row, one piece a lane) when the default
-// would give fewer workgroups than CUs: a small single GEMV then still spreads over the chip
-constexpr int R_SMALL = 4;
-
-// the grid of a launch with R rows a team: about gemv_blocks_per_cu workgroups per CU over the
-// whole batch, fewer when the rows run out (each wave then streams many row groups; its
-// activation registers are loaded once)
-inline int64_t gemv_blocks(const MMArgs& a, int fmt, int R, int L, int batch) {
-    const int64_t waves = (a.N + (int64_t)R * (64 / a.T) - 1) / ((int64_t)R * (64 / a.T));
-    int64_t blocks = (waves + 3) / 4;
-    int64_t cap = (int64_t)otpu_cu_count() * gemv_blocks_per_cu(L, fmt) / batch;
-    if (cap < 1) cap = 1;
-    return blocks > cap ? cap : blocks;
-}
-
 template <int FMT, int MR, int L, int R>
 void launch_grid(const MMArgs& a, int batch, hipStream_t s) {
     const int64_t blocks = gemv_blocks(a, FMT, R, L, batch);

@@ -7,6 +7,7 @@ Arrays: numpy in -> numpy out (copied through the device); device tensors stay o
 and every call is queued on the current torch stream."""
 from __future__ import annotations
 
+import functools
 from dataclasses import dataclass
 
 import numpy as np
@@ -193,13 +194,39 @@ def C_ptr(t, off: int):
     return ctypes.c_void_p(t.data_ptr() + off * t.element_size())
 
 
-# one activation row quantized inside the GEMV (otpu_mm_qin) instead of by a launch of its own: every
-# workgroup quantizes the row again, which pays while the weights are few (4096 x 1024 int4: one launch
-# of 4.7 us for two of 2.9 and 3.0; the LM head's 262144 rows: 160 us for 3 + 107)
-QIN_ROWS = 16384
-QIN_COLS = 16384                                          # columns otpu_mm_qin's prologue holds
-FOLD_COLS = 8192                                          # ... and otpu_mm_qin_fold's
+# One row's launches: QACT inside the GEMV (otpu_mm_qin, otpu_mm_qin_fold) saves a launch of ~3 us, and every
+# workgroup quantizes the whole row again.  So the columns they quantize together (otpu_qin_columns) decide.  Up
+# to 2.5M the single launch is the faster nearly everywhere (weight rows x columns, us, one / two launches: int4
+# 4096 x 1024 4.6 / 6.1, 6144 x 4096 (3.0M) 7.7 / 8.0, 16384 x 4096 14.3 / 11.4, 12288 x 16384 63 / 37; int8 4096 x
+# 4096 7.6 / 8.6, 12288 x 12288 59 / 39).  A fold of 256-column ranges: up to 8M (int4 1024 x 3072 5.8 / 10.5,
+# 8192 x 8192 28.8 / 24.8); of wider ones, whose sums a team's first lane adds one after another: up to 3M (2048
+# x 6144 11.4 / 11.5, 4096 x 6144 16.1 / 11.8).
+QIN_COLUMNS = 5 << 19
+FOLD_COLUMNS = 8 << 20
+WIDE_FOLD_COLUMNS = 3 << 20
 OFF_COLS = 1 << 24                                        # otpu_mm_dot's rows: 32-bit offsets over a tile's rows
+
+
+@functools.lru_cache(maxsize=4096)
+def _row_launch(fmt: str, N: int, K: int, width: int) -> bool:
+    """Whether one row's QACT and MM over ranges of `width` run as one launch."""
+    cols = X.load().otpu_qin_columns(K, width, N, X.FMT[fmt])
+    if width < K:
+        return 0 < cols <= (FOLD_COLUMNS if width == 256 else WIDE_FOLD_COLUMNS)
+    # (int8 rows of eight pieces a lane: the kernel's prologue is compiled for 16384 columns and leaves one wave
+    # a SIMD; 4096 x 8192 16.7 us against 11.7.  Past 8192 the other GEMV walks segments: 4096 x 10240 19.9 / 21.1)
+    return 0 < cols <= QIN_COLUMNS and not (fmt == "int8" and 6144 < K <= 8192)
+
+
+# ... and in ranges: the GEMV of every range and the sum of their rows (otpu_mm_ranges) in place of otpu_mm_dot's
+# tiles of 16 and 32 rows, where those are mostly padding and weights enough stream by.  One row (us, GEMV / tiles,
+# QACT in): int4 12288 x 8192 18.6 / 29.7, 2048 x 8192 10.6 / 12.7, 4096 x 1024 8.8 / 7.4; int8 2048 x 16384 13.9 /
+# 19.4, 2048 x 2048 9.7 / 8.5.  Two (without QACT): int4 12288 x 2048 12.2 / 16.9, 8192 x 2048 10.9 / 7.8.  Four: 70000
+# x 1024 int4 39.9 / 45.3, int8 34.0 / 29.0.
+def _stream_ranges(M: int, N: int, fmt: str, width: int) -> bool:
+    if M <= 2:
+        return N >= 12288 or (M == 1 and width >= 512)
+    return M <= 4 and fmt != "int8" and N >= 24576
 
 
 def _overlap(a, b) -> bool:
@@ -212,19 +239,16 @@ def _dot_row(x, w: QWeight, ranges, out) -> bool:
     """One fp32 row x (a contiguous device tensor [1, K]) @ w^T into out in one launch, QACT and the
     ranges' ACC chain inside; False where no such kernel takes the call, or out overlaps x (every
     workgroup reads the row while others store)."""
-    K, chunk = w.K, (D if w.fmt == "int8" else 2 * D)
-    if w.N > QIN_ROWS or x.data_ptr() % 16 or K % chunk or _overlap(x, out):
+    K, width = w.K, ranges[0]
+    if min(ranges) != max(ranges) or x.data_ptr() % 16 or not _row_launch(w.fmt, w.N, K, width) or _overlap(x, out):
         return False
     ws, srs = (0, 0) if w.srows is None else (w.srows.data_ptr(), w.srows.shape[1])
     fl = _flags(w.srows is None, w.rsc)
-    if len(ranges) == 1:
-        if K > QIN_COLS:
-            return False
+    if width == K:
         X.call("otpu_mm_qin", x.data_ptr(), None, None, None, 1, 0, K, K, w.rows.data_ptr(), w.rows.shape[1], ws, srs,
                w.N, X.FMT[w.fmt], fl, 0, out.data_ptr(), w.N, 0, X.stream())
         return True
-    width = ranges[0]
-    if fl or w.fmt == "int8" or K > FOLD_COLS or min(ranges) != max(ranges) or width % chunk:
+    if fl:
         return False
     X.call("otpu_mm_qin_fold", x.data_ptr(), None, None, None, K, width, w.rows.data_ptr(), w.rows.shape[1], ws, srs,
            w.N, X.FMT[w.fmt], 0, 0, out.data_ptr(), X.stream())
@@ -251,8 +275,9 @@ def dot(x, w: QWeight, acc=None, out=None, ranges=None, row_mode: bool = False, 
     4-bit formats need ranges that start on even blocks (a 128-byte chunk holds two blocks).
     rowmax: also return the row maxima of the final sums (MM RMAX on the last range).
 
-    Equal ranges run as one QACT launch and one MM launch (otpu_mm_dot: the ACC chain inside), one
-    fp32 row as a single launch where a kernel does both; anything else as a launch per range."""
+    Equal ranges run as one QACT launch and one MM launch (otpu_mm_dot: the ACC chain inside; few rows
+    on many weights otpu_mm_ranges), one fp32 row as a single launch where that is the faster; anything
+    else as a launch per range."""
     numpy_in = X.is_numpy(x)
     if acc is not None and out is not None:
         raise ValueError("dot: give either acc= or out=")
@@ -288,15 +313,24 @@ def dot(x, w: QWeight, acc=None, out=None, ranges=None, row_mode: bool = False, 
     al = X.dev(acc_scale, np.float32) if acc_scale is not None else None
     if one:
         s = X.stream()
+        R = len(ranges)
+        stream = R > 1 and al is None and R < 1 << 16 and _stream_ranges(M, N, w.fmt, width)
+        sizes = (4 * R * M * N,) if stream else ()
         if operand:
             qp, Sp, dp, act = q.data_ptr(), Sa[0].data_ptr(), da.data_ptr(), X.ACT_ANY
+            *part, _scr = _scratch(*sizes) if stream else (None,)
         else:                                             # the operand's three parts in one allocation
-            qp, Sp, dp, _scr = _scratch(M * K, 4 * M * len(ranges), M * (K // 32))
+            qp, Sp, dp, *part, _scr = _scratch(M * K, 4 * M * R, M * (K // 32), *sizes)
             act = X.ACT_ROW if row_mode else X.ACT_MX
             _qact_equal(xd, ranges, row_mode, qp, Sp, dp, s)
-        X.call("otpu_mm_dot", qp, K, Sp, dp, K // 32, M, K, width, w.rows.data_ptr(), w.rows.shape[1],
-               0 if unit else w.srows.data_ptr(), 0 if unit else w.srows.shape[1], N, X.FMT[w.fmt],
-               _flags(unit, w.rsc, acc is not None, al is not None), 0, act, X.ptr(al), y.data_ptr(), N, s)
+        ws, srs = (0, 0) if unit else (w.srows.data_ptr(), w.srows.shape[1])
+        fl = _flags(unit, w.rsc, acc is not None, al is not None)
+        if stream:
+            X.call("otpu_mm_ranges", qp, K, Sp, dp, K // 32, M, K, width, w.rows.data_ptr(), w.rows.shape[1], ws, srs, N,
+                   X.FMT[w.fmt], fl, 0, part[0], y.data_ptr(), N, s)
+        else:
+            X.call("otpu_mm_dot", qp, K, Sp, dp, K // 32, M, K, width, w.rows.data_ptr(), w.rows.shape[1], ws, srs, N,
+                   X.FMT[w.fmt], fl, 0, act, X.ptr(al), y.data_ptr(), N, s)
         return X.host(y) if numpy_in else y
     bpb = D if w.fmt == "int8" else D // 2
     rm = X.empty((M,), np.float32) if rowmax else None

@@ -83,3 +83,40 @@ def test_ranges_are_read_once(calls, M, fmt, widths):
         mxu.dot(torch.zeros((M, 1024)), weight(64, 1024, fmt), ranges=ranges)
         made.append([c[0] for c in calls])
     assert made[0] == made[1] == made[2] and made[0]
+
+
+def names(calls):
+    return [c[0][5:] for c in calls]
+
+
+@pytest.mark.skipif(not __import__("os").path.exists(X.LIB_PATH), reason="libotpu_amd.so not built")
+@pytest.mark.parametrize("fmt,N,K,width,want", [
+    ("int4", 4096, 1024, None, ["mm_qin"]), ("int4", 16384, 4096, None, ["qact", "mm_dot"]),
+    ("int8", 4096, 4096, None, ["mm_qin"]), ("int8", 64, 6400, None, ["qact", "mm_dot"]),
+    ("int8", 64, 8448, None, ["mm_qin"]), ("int8", 12288, 12288, None, ["qact", "mm_dot"]),
+    ("nvfp4", 64, 16384, None, ["mm_qin"]), ("nvfp4", 64, 16640, None, ["qact", "mm_dot"]),
+    ("int4", 64, 384, None, ["qact", "mm_dot"]),          # (an odd block count: half a chunk)
+    ("int4", 1024, 3072, 256, ["mm_qin_fold"]), ("int4", 8448, 8192, 256, ["qact_ranges", "mm_dot"]),
+    ("int4", 64, 8448, 256, ["qact_ranges", "mm_dot"]), ("int4", 64, 8448, 768, ["qact_ranges", "mm_ranges"]),
+    ("int4", 2048, 6144, 768, ["mm_qin_fold"]), ("int4", 4096, 6144, 768, ["qact_ranges", "mm_ranges"]),
+    ("int4", 64, 1024, 128, ["qact_ranges"] + ["mm"] * 8), ("int8", 64, 1024, 128, ["qact_ranges", "mm_dot"]),
+    ("int8", 12288, 512, 256, ["qact_ranges", "mm_ranges"]), ("int8", 12287, 512, 256, ["qact_ranges", "mm_dot"])])
+def test_one_rows_launches(calls, fmt, N, K, width, want):
+    mxu.dot(torch.zeros((1, K)), weight(N, K, fmt), ranges=None if width is None else [width] * (K // width))
+    assert names(calls) == want
+
+
+@pytest.mark.parametrize("M,fmt,N,want", [(2, "int4", 12287, "mm_dot"), (2, "int8", 12288, "mm_ranges"), (3, "int4", 12288, "mm_dot"),
+                                          (4, "nvfp4", 24576, "mm_ranges"), (4, "int8", 24576, "mm_dot"), (5, "int4", 24576, "mm_dot")])
+def test_few_rows_launches_in_ranges(calls, M, fmt, N, want):
+    w = weight(N, 512, fmt)
+    for x in (torch.zeros((M, 512)), operand(M, 512, [256, 256])):
+        calls.clear()
+        mxu.dot(x, w, ranges=[256, 256])
+        assert names(calls)[-1] == want
+        calls.clear()
+        mxu.dot(x, w, ranges=[256, 256], acc=torch.zeros((M, N)))
+        assert names(calls)[-1] == want
+    u = mxu.QWeight(w.rows, None, fmt, 512)               # (ASCALE: otpu_mm_ranges has none)
+    mxu.dot(torch.zeros((M, 512)), u, ranges=[256, 256], acc=torch.zeros((M, N)), acc_scale=torch.zeros(M))
+    assert names(calls)[-1] == "mm_dot"

@@ -126,3 +126,62 @@ def test_ranges_over_a_part_of_an_operand(mxu, fmt, M):
         want = CH.ranges_dot(host[:, :256 * R], (rows, srows), fmt, 256, mm=OC.mm)
         for S in (Sa[:R],) + ((Sa[:R, 0].contiguous(),) if M == 1 else ()):
             assert same_bits(mxu.dot((q, S, da, [256] * R), w).cpu().numpy(), want)
+
+
+def dot64(x, rows, srows, fmt, K, widths, old=None, row_mode=False):
+    """The oracle's dot: a QACT and an MM a range, the MMs' outputs added in range order."""
+    want, c0 = old, 0
+    bpb = 128 if fmt in ("int8", "rsc") else 64
+    for i, n in enumerate(widths):
+        q, Sa, da = OC.qact(np.ascontiguousarray(x[:, c0:c0 + n]), row_mode=row_mode)
+        kb = c0 // 128
+        want = OC.mm(q, Sa, da, np.ascontiguousarray(rows[:, kb * bpb:(kb + n // 128) * bpb]), srows, "int8" if fmt == "rsc" else fmt,
+                     n, flags=(MM.RSC if fmt == "rsc" else 0) | (MM.ACC if want is not None else 0),
+                     k0=0 if fmt == "rsc" else kb, old=want)
+        c0 += n
+    return want
+
+
+ONE = [(40, 256, None), (40, 384, None), (16384, 512, None), (16385, 512, None), (40, 6144, None), (40, 6400, None), (40, 8192, None),
+       (40, 8448, None), (70, 16384, None), (70, 16640, None), (2300, 4096, None), (6000, 4096, None),
+       (12287, 512, 256), (12288, 512, 256), (30, 8192, 256), (30, 8448, 256), (30, 8448, 768), (4096, 6144, 768), (50, 1024, 128),
+       (50, 1024, (512, 256, 256)), (50, 1024, (256, 512, 256))]
+
+
+@pytest.mark.parametrize("fmt", ["int8", "rsc", "int4", "fp4", "nvfp4"])
+def test_one_row_at_the_rules_edges(mxu, fmt):
+    """One row on both sides of each line of the rules that pick its launches; unequal ranges; a row whose
+    weights are half a chunk."""
+    import torch
+    rng = np.random.default_rng(3)
+    for N, K, width in ONE:
+        widths = [K] if width is None else list(width) if isinstance(width, tuple) else [width] * (K // width)
+        some = min(N, 64)
+        rows, srows = packed(rng, some, K, fmt)
+        rows, srows = np.resize(rows, (N, rows.shape[1])), np.resize(srows, (N, srows.shape[1]))
+        x = spread(rng, 1, K, 2.0, 32)
+        say("one row", fmt, N, K, width)
+        got = mxu.dot(torch.from_numpy(x).cuda(), qweight(mxu, rows, srows, fmt, K), ranges=widths).cpu().numpy()
+        want = dot64(x, np.ascontiguousarray(rows[:some]), np.ascontiguousarray(srows[:some]), fmt, K, widths)
+        assert same_bits(got, np.resize(want[0], (1, N))), (N, K, width)
+
+
+@pytest.mark.parametrize("M,fmt,N", [(1, "int8", 12288), (2, "int4", 12288), (2, "rsc", 12300), (3, "nvfp4", 24576), (4, "fp4", 24600),
+                                     (4, "int4", 24575)])
+def test_few_rows_on_many_weights_in_ranges(mxu, M, fmt, N):
+    """The GEMV of every range and the sum of their rows: overwriting, onto old values, from an operand."""
+    import torch
+    rng = np.random.default_rng(M + N)
+    K, width, some = 768, 256, 50
+    rows, srows = packed(rng, some, K, fmt)
+    w = qweight(mxu, np.resize(rows, (N, rows.shape[1])), np.resize(srows, (N, srows.shape[1])), fmt, K)
+    x = spread(rng, M, K, 2.0, 32)
+    xd = torch.from_numpy(x).cuda()
+    old = np.resize(rng.standard_normal((M, some)).astype(np.float32), (M, some))
+    idx = np.arange(N) % some
+    say("few rows", M, fmt, N)
+    want = dot64(x, rows, srows, fmt, K, [width] * 3)[:, idx]
+    assert same_bits(mxu.dot(xd, w, ranges=[width] * 3).cpu().numpy(), want)
+    assert same_bits(mxu.dot(mxu.quantize_ranges(xd, [width] * 3), w).cpu().numpy(), want)
+    acc = torch.from_numpy(np.ascontiguousarray(old[:, idx])).cuda()
+    assert same_bits(mxu.dot(xd, w, acc=acc, ranges=[width] * 3).cpu().numpy(), dot64(x, rows, srows, fmt, K, [width] * 3, old)[:, idx])
