@@ -5,6 +5,7 @@
 #include <cstdlib>
 
 #include "gemv_args.h"
+#include "prefill_args.h"
 
 namespace otpu {
 
@@ -184,26 +185,66 @@ int otpu_prefill_try(const int8_t* q, int64_t ldq, const float* Sa, const uint8_
                      int ranges, const uint8_t* w, int64_t rs, const uint8_t* ws, int64_t srs, int N, int fmt, int flags,
                      int k0, const float* alpha, float* out, int64_t ors, hipStream_t s);
 
-// MM of several activation rows on the MFMA kernels, over `ranges` equal column ranges (their ACC
-// chain): 0 or an error, or > 0 where none of them takes the call (RMAX, offset rows that are not
-// whole words: the GEMV then streams it, a few rows a launch).  act: what is known of the activation
-// offsets (OTPU_ACT_*).  The kernels give the same bits; the lines between them, measured (us):
-//   the batch kernel (no LDS; K split over waves) below 3/4 of a 32 x 128 tile a CU: int8 1024 x 2048
-//     weights at 512 rows 19.2 against the prefill kernel's 19.5, 4096 x 1024 at 128 rows 12.7 / 12.3
-//     (128 tiles), int4 12288 x 2048 at 50 rows 29 / 28 (192 tiles), at 128 rows 48 / 31 (384)
-//   the GEMMs (128 x 128 tiles, one a CU at a time) for plain int8 and 4-bit weights: with one
-//     activation offset they multiply folded operands with no work a product (4096 x 2048 x 8192: rsc
-//     116, int4 214 against the prefill kernel's 161, 308), with several they are the slower (int4
-//     395 / 309).  So they run where the offsets are one (ROW) or unknown, and their last round of
+// Whether the 128 x 128 GEMM is faster than the prefill kernel on activations of one offset, where it multiplies
+// folded operands with no work a product: us a round of tiles and of its start, and per 128 columns, fitted to
+// 409 shapes a format (the kernel these lines choose is within 0.5% of the fastest on the mean, plain int8 1.1%).
+// GEMM / prefill: int4 512 x 2048 x 8192 32 / 46, 1000 x 6144 x 2048 72 / 78, 300 x 2048 x 12288 60 / 46; int8 (RSC)
+// 384 x 8192 x 8192 35 / 61, 700 x 2048 x 1024 19 / 14.  An int8 tile whose activation rows end inside it stores a
+// value at a time, 6 us a round of such: every round of an XCD's where its tiles all are (workgroup b runs on XCD
+// b % 8, row tiles innermost: 1000 x 2048 x 8192 38.5, 1024 rows 26).
+struct RowCost {
+    double gemm, gemm_k, ragged;                          // a round of GEMM tiles
+    double start, start_k, tile, tile_k;                  // the prefill kernel's start, a round of 32-row tiles
+};
+static bool gemm_pays(int M, int N, int K, int fmt, bool plain) {
+    static const RowCost costs[4] = {{6.0, 0.44, 6.0, 4.7, 0.27, 1.2, 0.30},      // int8 (plain only)
+                                     {9.3, 1.23, 0.0, 5.3, 0.44, 1.3, 0.55},      // int4, fp4
+                                     {9.5, 1.43, 0.0, 5.7, 0.58, 1.6, 0.80},      // nvfp4
+                                     {6.5, 0.88, 0.0, 5.3, 0.44, 1.3, 0.55}};     // 4-bit UNIT / RSC: one plane
+    const RowCost& c = costs[fmt == OTPU_INT8 ? 0 : plain ? 3 : fmt == OTPU_NVFP4 ? 2 : 1];
+    const int tm = (M + 127) / 128, all = (tm & -tm) < 8 ? tm & -tm : 8;          // gcd(tm, 8)
+    const double kb = K / OTPU_D, ragged = M % 128 ? c.ragged * all / tm : 0.0;
+    const double gemm = (double)pf::rounds(M, N, 128) * (c.gemm + c.gemm_k * kb + ragged);
+    const double tiles = pf::row_tiles(M, N, fmt, 1) == 2 ? 1.7 * pf::rounds(M, N, 64) : (double)pf::rounds(M, N, 32);
+    return gemm < c.start + c.start_k * kb + tiles * (c.tile + c.tile_k * kb);
+}
+
+// MM of several activation rows, over `ranges` equal column ranges (their ACC chain): 0 or an error, or > 0
+// where none of these kernels takes the call (RMAX, offset rows that are not whole words: the GEMV then
+// streams it, a few rows a launch).  act: what is known of the activation offsets (OTPU_ACT_*).  The kernels
+// give the same bits; the lines between them, measured (M x K x N, us):
+//   the GEMV, its rows in two passes, for 5 and 6 rows on many 4-bit weights of one or two pieces a lane: int4 5 x
+//     4096 x 40000 38 against 48 (batch) and 56 (prefill), 6 x 2048 x 28672 21 / 18 / 24, nvfp4 5 x 2048 x 20000 21 / 28
+//   the batch kernel (no LDS; K split over waves) below 9/16 of a 32 x 128 tile a CU, 3/4 for up to 16 rows:
+//     batch / prefill int4 64 x 2048 x 8192 (128 tiles) 17.5 / 22.7, 300 x 6144 x 2048 (160) 60 / 56, int8 33 x 8192 x
+//     8192 (128) 38 / 70, nvfp4 32 x 1024 x 20000 (157) 28.9 / 18.6; plain int8 16 x 1024 x 20000 13.5 / 9.8, and with one
+//     offset, where the GEMM starts sooner, below 5/16: 384 x 2048 x 1024 (96) 16.3 / 12.3
+//   the GEMM for plain int8 and 4-bit weights: with one activation offset (ROW) where it pays (above); with several
+//     it is the slower (int4 4096 x 2048 x 8192 376 / 295; two offsets of plain int8 alone are the faster there, by
+//     up to 1.5, and three the slower by up to 1.3); with offsets unknown where it would pay and its last round of
 //     tiles is at least 4/5 full
 //   the prefill kernel for the rest
 static int mm_rows(const int8_t* q, int64_t ldq, const float* Sa, const uint8_t* da, int64_t ldda, int M, int K,
                    int ranges, const uint8_t* w, int64_t rs, const uint8_t* ws, int64_t srs, int N, int fmt, int flags,
                    int k0, int act, const float* alpha, float* out, int64_t ors, hipStream_t s) {
-    const int64_t n128 = (N + 127) / 128, tiles = (M + 127) / 128 * n128, cus = otpu_cu_count();
-    if ((M + 31) / 32 * n128 < cus * 3 / 4)
+    if (flags & OTPU_RMAX) return 1;
+    const bool plain = (flags & (OTPU_UNIT | OTPU_RSC)) != 0, int8 = fmt == OTPU_INT8;
+    const int64_t n128 = (N + 127) / 128, cus = otpu_cu_count();
+    if (ranges == 1 && M <= 6 && !int8 && K >= 2048 && n128 >= cus * 9 / 16 && n128 <= cus * 5 / 2) {
+        int T, L;
+        pick_team(K / 32, &T, &L);
+        if (L <= 2) {
+            MMArgs a = make_args(q, ldq, Sa, da, ldda, M, K, w, rs, ws, srs, N, flags, k0);
+            a.alpha = alpha; a.out = out; a.ors = ors;
+            return launch_gemv(a, fmt, 1, s);
+        }
+    }
+    const bool plain8 = int8 && plain && ranges == 1;
+    const int64_t sixteenths = M <= 16 ? (plain8 ? 9 : 12) : plain8 && act == OTPU_ACT_ROW ? 5 : 9;
+    if ((M + 31) / 32 * n128 < cus * sixteenths / 16)
         return otpu_batch_try(q, ldq, Sa, da, ldda, M, K, ranges, w, rs, ws, srs, N, fmt, flags, k0, alpha, out, ors, s);
-    if (ranges == 1 && act != OTPU_ACT_MX && tiles * 5 / 4 >= (tiles + cus - 1) / cus * cus) {
+    if (ranges == 1 && (!int8 || plain) && act != OTPU_ACT_MX && gemm_pays(M, N, K, fmt, plain) &&
+        (act == OTPU_ACT_ROW || (M + 127) / 128 * n128 * 5 / 4 >= pf::rounds(M, N, 128) * cus)) {
         int rc = otpu_gemm_try(q, ldq, Sa, da, ldda, M, K, w, rs, ws, srs, N, fmt, flags, k0, alpha, out, ors, s);
         if (rc <= 0) return rc;
         rc = otpu_gemm4_try(q, ldq, Sa, da, ldda, M, K, w, rs, ws, srs, N, fmt, flags, k0, alpha, out, ors, s);

@@ -14,18 +14,17 @@ int otpu_prefill_try(const int8_t* q, int64_t ldq, const float* Sa, const uint8_
     a.w = w; a.rs = rs; a.ws = ws; a.srs = srs; a.N = N; a.flags = flags;
     a.k0 = (flags & (OTPU_UNIT | OTPU_RSC)) ? 0 : k0;
     a.alpha = alpha; a.out = out; a.ors = ors; a.ranges = ranges;
-    // 64 rows a tile where that still makes two workgroups a CU, else 32 (int4 2000 x 1024 x 4096: 50
-    // against 54 us; 512 x 2048 x 1024: 30 against 22; nvfp4 1999 x 6144 x 2048 in ranges of 768: 222 against 280)
-    const int64_t t64 = (int64_t)((M + 63) / 64) * ((N + 127) / 128);
-    const int ms = t64 >= 2 * otpu_cu_count() ? 2 : 1;
+    const int ms = pf::row_tiles(M, N, fmt, ranges);
     a.tiles_m = (M + 32 * ms - 1) / (32 * ms);
     a.tiles_n = (N + 127) / 128;
     a.vec4 = ((uintptr_t)out % 16 == 0) && (ors % 4 == 0);
+    bool ok;
     switch (fmt) {
-        case OTPU_INT8: pf::launch_fmt<OTPU_INT8>(a, ms, s); break;
-        case OTPU_INT4: pf::launch_fmt<OTPU_INT4>(a, ms, s); break;
-        case OTPU_FP4: pf::launch_fmt<OTPU_FP4>(a, ms, s); break;
-        default: pf::launch_fmt<OTPU_NVFP4>(a, ms, s); break;
+        case OTPU_INT8: ok = pf::launch_fmt<OTPU_INT8>(a, ms, s); break;
+        case OTPU_INT4: ok = pf::launch_fmt<OTPU_INT4>(a, ms, s); break;
+        case OTPU_FP4: ok = pf::launch_fmt<OTPU_FP4>(a, ms, s); break;
+        default: ok = pf::launch_fmt<OTPU_NVFP4>(a, ms, s); break;
     }
+    if (!ok) return otpu_fail(OTPU_EINVAL, "mm prefill: no kernel of format %d for %d rows a tile in ranges", fmt, 32 * ms);
     return otpu_launch_check("mm prefill");
 }

@@ -21,8 +21,25 @@ struct Args {
     int vec4;                       // out 16-byte aligned and ors a multiple of 4: float4 stores
 };
 
+// rounds of tiles of `rows` x 128 rows, one tile a CU
+inline int64_t rounds(int M, int N, int rows) {
+    const int64_t tiles = (int64_t)((M + rows - 1) / rows) * ((N + 127) / 128), cus = otpu_cu_count();
+    return (tiles + cus - 1) / cus;
+}
+
+// row tiles of 32 a workgroup, 1 or 2.  A round of 64 rows costs ~1.7 of 32's, and a call a round's start besides
+// (us at 32 -> at 64 rows a tile: int4 512 x 2048 x 8192 52.5 -> 46.1, 300 rows 40.8 -> 44.1, 64 rows 22.7 -> 30.9;
+// nvfp4 2 x 1024 x 70000 in ranges 51.8 -> 82.7): this line is within 0.3% of the faster one on the mean of 818
+// shapes.  int8's ranges take 32 rows (65 x 2048 x 12288 45 / 71, 512 x 2048 x 8192 80 / 79): no kernel of 64
+constexpr bool has_tall_tile(int fmt, bool ranged) { return !(fmt == OTPU_INT8 && ranged); }
+inline int row_tiles(int M, int N, int fmt, int ranges) {
+    if (!has_tall_tile(fmt, ranges > 1)) return 1;
+    return 5 * (1 + rounds(M, N, 32)) > 8 * (1 + rounds(M, N, 64)) ? 2 : 1;
+}
+
+// false: no such kernel (nothing launched)
 template <int FMT>
-void launch_fmt(const Args& a, int ms, hipStream_t s);
+bool launch_fmt(const Args& a, int ms, hipStream_t s);
 
 }  // namespace pf
 }  // namespace otpu

@@ -637,15 +637,19 @@ __global__ __launch_bounds__(256, 2) void prefill_kernel(Args p) {
 }
 
 template <int FMT>
-void launch_fmt(const Args& a, int ms, hipStream_t s) {
+bool launch_fmt(const Args& a, int ms, hipStream_t s) {
     const unsigned grid = (unsigned)(a.tiles_m * a.tiles_n);
-    if (a.ranges > 1) {
-        if (ms == 1) prefill_kernel<FMT, 1, true><<<grid, 256, 0, s>>>(a);
-        else prefill_kernel<FMT, 2, true><<<grid, 256, 0, s>>>(a);
-    } else {
+    if (a.ranges == 1) {
         if (ms == 1) prefill_kernel<FMT, 1, false><<<grid, 256, 0, s>>>(a);
         else prefill_kernel<FMT, 2, false><<<grid, 256, 0, s>>>(a);
+        return true;
     }
+    if (ms == 1) {
+        prefill_kernel<FMT, 1, true><<<grid, 256, 0, s>>>(a);
+        return true;
+    }
+    if constexpr (has_tall_tile(FMT, true)) prefill_kernel<FMT, 2, true><<<grid, 256, 0, s>>>(a);
+    return has_tall_tile(FMT, true);
 }
 
 #undef INL

@@ -3,6 +3,6 @@
 
 namespace otpu {
 namespace pf {
-template void launch_fmt<OTPU_NVFP4>(const Args& a, int ms, hipStream_t s);
+template bool launch_fmt<OTPU_NVFP4>(const Args& a, int ms, hipStream_t s);
 }  // namespace pf
 }  // namespace otpu

@@ -77,12 +77,42 @@ def test_batch(X, M, N, K, fmt, wk, ak):
 @pytest.mark.parametrize("fmt,wk,ak", KINDS + [("int8", "rsc", "mx"), ("int8", "rsc", WIN), ("int8", "x8", "row"),
                                                ("fp4", "x4", "row"), ("nvfp4", "x4", "row")])
 def test_prefill(X, M, N, K, act, fmt, wk, ak):
-    """act 2: the prefill kernel (32 and 64 rows a tile); 0 and 1: the GEMMs, ragged last tiles."""
+    """The prefill kernel (32 and 64 rows a tile), and 4-bit weights on the GEMM where offsets are unknown."""
     rng = np.random.default_rng(M + N + K)
     q, Sa, da, rows, srows, fl = operands(rng, M, N, K, fmt, wk, ak)
     say("prefill", M, N, K, act, fmt, wk, ak)
     got = mm_dot(X, q, Sa, da, rows, srows, fmt, K, K, fl, act=act)
     assert same_bits(got, OC.mm(q, Sa, da, rows, srows, fmt, K, flags=fl))
+
+
+@pytest.mark.parametrize("M,N,K,act", [(500, 8100, 2048, 0), (300, 8100, 2048, 1), (129, 16200, 2048, 1)])
+@pytest.mark.parametrize("fmt,wk,ak", [("int8", "rsc", "row"), ("int8", "rsc", "mx"), ("int8", "unit", (0, 3)), ("int8", "rsc", (0, 20)),
+                                       ("int4", "x4", "row"), ("int4", "spread", WIN), ("int4", "rsc", "row"), ("fp4", "x4", "row"),
+                                       ("fp4", "wide", "mx"), ("nvfp4", "x4", "row"), ("nvfp4", "tiny", "mx")])
+def test_gemm_ragged_tiles(X, M, N, K, act, fmt, wk, ak):
+    """Calls the rule sends to the 128 x 128 GEMMs (their offsets unknown, or said to be one), whose last tiles
+    end inside; activations of any offsets (the walk in the GEMMs)."""
+    rng = np.random.default_rng(M + N)
+    q, Sa, da, rows, srows, fl = operands(rng, M, 60, K, fmt, wk, ak)
+    say("gemm ragged", M, N, K, act, fmt, wk, ak)
+    rep = lambda a: np.resize(a, (N, a.shape[1]))  # noqa: E731
+    got = mm_dot(X, q, Sa, da, rep(rows), rep(srows), fmt, K, K, fl, act=act)
+    want = OC.mm(q, Sa, da, rows, srows, fmt, K, flags=fl)
+    assert same_bits(got, want[:, np.arange(N) % 60])
+
+
+@pytest.mark.parametrize("M,N,K", [(5, 18305, 2048), (6, 18304, 4096), (7, 18305, 2048), (5, 18305, 2304), (16, 20000, 256), (17, 18400, 256)])
+@pytest.mark.parametrize("fmt,wk,ak", [("int8", "rsc", "mx"), ("int8", "spread", "mx"), ("int4", "x4", "mx"), ("nvfp4", "x4", WIN)])
+def test_few_rows_on_many_weights(X, M, N, K, fmt, wk, ak):
+    """Both sides of the lines between the GEMV, the batch and the prefill kernel, onto old values."""
+    rng = np.random.default_rng(M + K)
+    q, Sa, da, rows, srows, fl = operands(rng, M, 60, K, fmt, wk, ak)
+    old = rng.standard_normal((M, 60)).astype(np.float32)
+    idx = np.arange(N) % 60
+    rep = lambda a: np.resize(a, (N, a.shape[1]))  # noqa: E731
+    say("few rows", M, N, K, fmt, wk, ak)
+    got = mm_dot(X, q, Sa, da, rep(rows), rep(srows), fmt, K, K, fl | MM.ACC, act=2, old=np.ascontiguousarray(old[:, idx]))
+    assert same_bits(got, OC.mm(q, Sa, da, rows, srows, fmt, K, flags=fl | MM.ACC, old=old)[:, idx])
 
 
 @pytest.mark.parametrize("fmt,lo,hi", [("int4", 0x88, 0x77), ("nvfp4", 0xFF, 0x77)])
