@@ -1,9 +1,9 @@
-"""The 4-bit prefill GEMM (int4x / fp4x6 / nvfp4 weights, and their RSC / UNIT forms, on the int8
-MFMA units: csrc/gemm4.hip) against the C oracle bit for bit: single activation planes (ROW),
-several (MX, Horner over the planes), offsets past the window, weight blocks whose offsets spread
-(the folded multipliers), nvfp4's per-16-group E4M3 scales (subnormal ones included), tiles the
-bounds refuse (the exact VALU path), ACC / ASCALE, k0 column slices, ragged tiles, and the c3
-shape at full size (`opentpu/isasim.py:749-910`)."""
+"""MM of several rows with 4-bit weights (int4x / fp4x6 / nvfp4, and their RSC / UNIT forms) against the C
+oracle bit for bit (`opentpu/isasim.py:749-910`): activations of one offset (ROW), of several (MX), offsets
+past the window, weight blocks whose offsets spread, nvfp4's per-16-group E4M3 scales (subnormal ones
+included), ACC / ASCALE, k0 column slices, ragged tiles, and the c3 shape at full size.  The c3 shape runs
+the 128 x 128 GEMM (csrc/gemm4.hip); the small cases are below its line and run the batch kernel
+(csrc/batch_impl.h), and test_gpu_rows.py's test_gemm_kinds runs the same kinds on the GEMM."""
 import sys
 
 import numpy as np
@@ -80,8 +80,8 @@ CASES = [  # M, N, K, fmt, weights (x4 | spread | wide | rsc | unit), activation
     (48, 130, 6144, "fp4", "spread", "row", 0),
     (16, 8192, 256, "int4", "x4", "row", 0),        # 64 column tiles: the XCD-major order
     (17, 1000, 128, "fp4", "x4", "mx", 0),
-    (128, 128, 2048, "int4", "x4", "wide", 0),      # activation offsets past the Horner bound: VALU
-    (80, 96, 1024, "fp4", "wide", "row", 0),        # weight offsets past the folding range: VALU
+    (128, 128, 2048, "int4", "x4", "wide", 0),      # activation offsets past the Horner bound
+    (80, 96, 1024, "fp4", "wide", "row", 0),        # weight offsets past the folding range
     (200, 256, 1024, "int4", "x4", (0, 1, 2), 0),
     (200, 256, 1024, "fp4", "x4", (0, 20), 0),      # offsets past the window: those groups drop
     (200, 256, 1024, "int4", "x4", (2, 5, 9), 0),   # drops where d + dw > 11
@@ -96,8 +96,8 @@ CASES = [  # M, N, K, fmt, weights (x4 | spread | wide | rsc | unit), activation
     (50, 64, 384, "nvfp4", "spread", "row", 0),     # three K stages
     (130, 257, 640, "nvfp4", "tiny", "mx", 0),      # subnormal scales: those groups always drop
     (80, 96, 1024, "nvfp4", "wide", "row", 0),
-    (80, 96, 1024, "nvfp4", "wider", "row", 0),     # scales past the folding range: VALU
-    (128, 128, 2048, "nvfp4", "x4", "wide", 0),     # activation offsets past the Horner bound: VALU
+    (80, 96, 1024, "nvfp4", "wider", "row", 0),     # scales past the folding range
+    (128, 128, 2048, "nvfp4", "x4", "wide", 0),     # activation offsets past the Horner bound
     (200, 256, 1024, "nvfp4", "x4", (0, 20), 0),    # offsets past the window: those groups drop
     (200, 256, 1024, "nvfp4", "x4", (2, 5, 9, 13), 0),   # drops where d + dw > 13
     (16, 8192, 256, "nvfp4", "x4", "row", 0),       # 64 column tiles: the XCD-major order

@@ -10,6 +10,7 @@ from conftest import same_bits
 from oracle import cpu as OC
 from oracle import fp32 as F
 from oracle import mm as MM
+from test_gpu_gemm4 import CASES as GEMM4_CASES
 from test_gpu_gemm4 import activations, say, weights
 
 pytestmark = pytest.mark.gpu
@@ -99,6 +100,38 @@ def test_gemm_ragged_tiles(X, M, N, K, act, fmt, wk, ak):
     got = mm_dot(X, q, Sa, da, rep(rows), rep(srows), fmt, K, K, fl, act=act)
     want = OC.mm(q, Sa, da, rows, srows, fmt, K, flags=fl)
     assert same_bits(got, want[:, np.arange(N) % 60])
+
+
+GEMM_KINDS = [c for c in GEMM4_CASES] + [(0, 0, K, "int8", wk, ak, 0) for K, wk, ak in [
+    (1024, "rsc", "row"), (640, "unit", "row"), (128, "rsc", "row"), (4096, "rsc", "mx"), (8192, "rsc", "mx"), (6144, "rsc", "row"),
+    (256, "rsc", "row"), (128, "unit", "mx"), (1024, "rsc", (0, 1)), (1024, "rsc", (0, 1, 2)), (1024, "rsc", (1, 3, 4)),
+    (1024, "rsc", (0, 20)), (1024, "rsc", (2, 5, 17)), (1024, "unit", (0, 31)), (4096, "rsc", (0, 1)), (4224, "rsc", (0, 2)),
+    (8192, "rsc", (1,)), (512, "rsc", (20, 30)), (2048, "unit", "wide")]]
+
+
+@pytest.mark.parametrize("M0,N0,K,fmt,wk,ak,k0", GEMM_KINDS)
+def test_gemm_kinds(X, M0, N0, K, fmt, wk, ak, k0):
+    """The kinds of weights, offsets and K of the small GEMM cases (test_gpu_gemm4.py, test_gpu_parity.py: so few
+    rows and columns run the batch kernel) at sizes that the rule sends to the GEMMs: a round of 128 x 128 tiles
+    where the prefill kernel has three or four, the call saying that its offsets are one, which picks a kernel and
+    changes no bit.  One row tile (its rows ending inside it unless K is short), or four."""
+    M, N = ((128 if K < 512 else 100), 31990) if K <= 2048 else (500, 8190)
+    rng = np.random.default_rng(K + len(wk))
+    q, Sa, da = activations(rng, M, K, ak)
+    if fmt == "int8":
+        rows, srows = int8_weights(rng, 60, K, "rsc")
+    else:
+        rows, srows = weights(rng, 60, K, fmt, wk, k0)
+    fl = {"rsc": MM.RSC, "unit": MM.UNIT}.get(wk, 0)
+    rep = lambda a: np.resize(a, (N, a.shape[1]))  # noqa: E731
+    idx = np.arange(N) % 60
+    say("gemm kinds", M, N, K, fmt, wk, ak, k0)
+    got = mm_dot(X, q, Sa, da, rep(rows), rep(srows), fmt, K, K, fl, k0=k0, act=1)
+    assert same_bits(got, OC.mm(q, Sa, da, rows, srows, fmt, K, flags=fl, k0=k0)[:, idx])
+    if K in (512, 640, 1024):                             # onto old values
+        old = rng.standard_normal((M, 60)).astype(np.float32)
+        got = mm_dot(X, q, Sa, da, rep(rows), rep(srows), fmt, K, K, fl | MM.ACC, k0=k0, act=1, old=np.ascontiguousarray(old[:, idx]))
+        assert same_bits(got, OC.mm(q, Sa, da, rows, srows, fmt, K, flags=fl | MM.ACC, k0=k0, old=old)[:, idx])
 
 
 @pytest.mark.parametrize("M,N,K", [(5, 18305, 2048), (6, 18304, 4096), (7, 18305, 2048), (5, 18305, 2304), (16, 20000, 256), (17, 18400, 256)])
