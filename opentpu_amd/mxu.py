@@ -167,9 +167,22 @@ def _qact_equal(xd, ranges, row_mode: bool, q: int, Sa: int, da: int, stream) ->
         X.call("otpu_qact", xd.data_ptr(), M, K, K, 32, fl, None, None, q, K, Sa, da, K // 32, None, 0, stream)
 
 
+class Operand(tuple):
+    """(q, Sa, da, ranges) as quantize_ranges returns it, with its mode: the offsets of a ROW operand are all 0.
+    A dot picks a kernel by it (a plain tuple's offsets are unknown); no bit of its result depends on it."""
+    row = False
+
+
+def _operand(q, Sa, da, ranges, row: bool) -> Operand:
+    op = Operand((q, Sa, da, ranges))
+    op.row = row
+    return op
+
+
 def quantize_ranges(x, ranges=None, row_mode: bool = False):
     """QACT of x [M, K] in column ranges (widths summing to K, each a multiple of 128; default
-    one range): the int8 operand [M, K], Sa per range [n_ranges, M], da [M, K/32]."""
+    one range): the int8 operand [M, K], Sa per range [n_ranges, M], da [M, K/32] and the ranges (an
+    Operand)."""
     xd = X.dev(x, np.float32)
     M, K = xd.shape
     ranges = _check_ranges(ranges, K)
@@ -178,7 +191,7 @@ def quantize_ranges(x, ranges=None, row_mode: bool = False):
     Sa = X.empty((len(ranges), M), np.float32)
     if min(ranges) == max(ranges):
         _qact_equal(xd, ranges, row_mode, q.data_ptr(), Sa.data_ptr(), da.data_ptr(), X.stream())
-        return q, Sa, da, ranges
+        return _operand(q, Sa, da, ranges, bool(row_mode))
     flags = X.Q_ROW if row_mode else 0
     c0 = 0
     for i, w in enumerate(ranges):
@@ -186,7 +199,7 @@ def quantize_ranges(x, ranges=None, row_mode: bool = False):
         X.call("otpu_qact", X.ptr(xs), M, w, K, 32, flags, None, None, C_ptr(q, c0), K,
                X.ptr(Sa[i]), C_ptr(da, c0 // 32), K // 32, None, 0, X.stream())
         c0 += w
-    return q, Sa, da, ranges
+    return _operand(q, Sa, da, ranges, bool(row_mode))
 
 
 def C_ptr(t, off: int):
@@ -267,6 +280,17 @@ def _scratch(*sizes):
     return *(p + o for o in offs), t
 
 
+def _operand_act(x, w: QWeight) -> int:
+    """What an operand's mode says of its offsets to otpu_mm_dot.  Of MX offsets and plain weights (RSC, UNIT)
+    nothing is said: two a tile are the faster on the GEMM (int8 512 x 2048 x 8192 21 us against 32), three not
+    (33.5 / 32.3); on 4-bit weights with scale rows either is the slower there (int4 51.9 and 48.1 / 46.1)."""
+    if not isinstance(x, Operand):
+        return X.ACT_ANY
+    if x.row:
+        return X.ACT_ROW
+    return X.ACT_ANY if w.fmt == "int8" or w.rsc or w.srows is None else X.ACT_MX
+
+
 def dot(x, w: QWeight, acc=None, out=None, ranges=None, row_mode: bool = False, rowmax: bool = False,
         acc_scale=None):
     """x [M, K] (fp32, quantized here, or a (q, Sa, da, ranges) operand from quantize_ranges)
@@ -317,7 +341,7 @@ def dot(x, w: QWeight, acc=None, out=None, ranges=None, row_mode: bool = False, 
         stream = R > 1 and al is None and R < 1 << 16 and _stream_ranges(M, N, w.fmt, width)
         sizes = (4 * R * M * N,) if stream else ()
         if operand:
-            qp, Sp, dp, act = q.data_ptr(), Sa[0].data_ptr(), da.data_ptr(), X.ACT_ANY
+            qp, Sp, dp, act = q.data_ptr(), Sa[0].data_ptr(), da.data_ptr(), _operand_act(x, w)
             *part, _scr = _scratch(*sizes) if stream else (None,)
         else:                                             # the operand's three parts in one allocation
             qp, Sp, dp, *part, _scr = _scratch(M * K, 4 * M * R, M * (K // 32), *sizes)

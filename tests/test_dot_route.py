@@ -120,3 +120,17 @@ def test_few_rows_launches_in_ranges(calls, M, fmt, N, want):
     u = mxu.QWeight(w.rows, None, fmt, 512)               # (ASCALE: otpu_mm_ranges has none)
     mxu.dot(torch.zeros((M, 512)), u, ranges=[256, 256], acc=torch.zeros((M, N)), acc_scale=torch.zeros(M))
     assert names(calls)[-1] == "mm_dot"
+
+
+@pytest.mark.parametrize("fmt", ["int8", "int4"])
+def test_an_operands_mode_picks_the_kernel(calls, fmt):
+    """quantize_ranges' operand says whether its offsets are one; parts put together by hand say nothing."""
+    w = weight(64, 512, fmt)
+    for row in (True, False):
+        op = mxu.quantize_ranges(torch.zeros((6, 512)), None, row)
+        assert isinstance(op, tuple) and len(op) == 4 and op[3] == [512]
+        for x, act in ((op, X.ACT_ROW if row else X.ACT_ANY if fmt == "int8" else X.ACT_MX), (tuple(op), X.ACT_ANY),
+                       (op[:3] + ([512],), X.ACT_ANY)):
+            calls.clear()
+            mxu.dot(x, w)
+            assert names(calls) == ["mm_dot"] and calls[0][17] == act
