@@ -172,12 +172,10 @@ def lm_head(steps, warmup):
     return ms, int(tok.item()), ms_pick, ms_both, sample
 
 
-def gemm(steps, warmup, row_mode=True, fmt="int8", generic=False):
+def gemm(steps, warmup, row_mode=True, fmt="int8"):
     """The c3 prefill GEMM, RSC weights (fmt int8) or 4-bit group-quantized ones (int4x / fp4x6 / nvfp4:
     the 4-bit GEMM); activations ROW-quantized (the headline: one scale a row, a single exact
-    plane) or MX (group offsets: several planes).  generic: the int8 GEMM's generic copy on the
-    same operands instead of the one compiled for c3's sizes and strides (OTPU_GENERIC_COPIES
-    set while the step is captured; the same work and results)."""
+    plane) or MX (group offsets: several planes)."""
     import torch
 
     from opentpu_amd import _lib as X
@@ -194,17 +192,16 @@ def gemm(steps, warmup, row_mode=True, fmt="int8", generic=False):
     def step():
         X.call("otpu_mm", X.ptr(q), K, X.ptr(Sa), X.ptr(da), K // 32, M, K, X.ptr(rows), rows.shape[1], X.ptr(srows),
                srows.shape[1], N, X.FMT[fmt], fl, 0, None, X.ptr(out), N, None, X.stream())
-    with generic_copies(generic):
-        ms = timed(step, steps, warmup, torch.cuda.current_stream())
+    ms = timed(step, steps, warmup, torch.cuda.current_stream())
     sample = tuple(t.cpu().numpy() for t in (q, Sa, da, rows, srows, out))
     return ms, sample
 
 
 @contextlib.contextmanager
 def generic_copies(on):
-    """OTPU_GENERIC_COPIES set inside (when on): the library then launches its generic kernel
-    copies instead of the ones compiled for the c3 / c4 shapes (read per GEMM call and when a
-    chain's plan is built; the same work and results)."""
+    """OTPU_GENERIC_COPIES set inside (when on): the persistent step then runs its generic kernel
+    copy instead of the one compiled for its shape (read when a chain's plan is built; the same work
+    and results)."""
     old = os.environ.get("OTPU_GENERIC_COPIES")
     if on:
         os.environ["OTPU_GENERIC_COPIES"] = "1"
@@ -471,9 +468,9 @@ def main():
     ap.add_argument("--warmup", type=int, default=5)
     ap.add_argument("--batch", type=int, default=80)
     ap.add_argument("--no-cpu", action="store_true")
-    ap.add_argument("--only", default="", help="comma list of c1,c2s,c3,c3r,c3m,c3q,c3g,c3blas,c4,c5,copy (default: "
-                    "c1,c2s,c3,c4,c5; c3r / c3m: the ROW / the MX int8 GEMM alone; c3q: the 4-bit GEMMs alone; c3g: "
-                    "the ROW GEMM's generic copy; c3blas: hipBLASLt's int8 GEMM at c3's shape, a yardstick); "
+    ap.add_argument("--only", default="", help="comma list of c1,c2s,c3,c3r,c3m,c3q,c3blas,c4,c5,copy (default: "
+                    "c1,c2s,c3,c4,c5; c3r / c3m: the ROW / the MX int8 GEMM alone; c3q: the 4-bit GEMMs alone; "
+                    "c3blas: hipBLASLt's int8 GEMM at c3's shape, a yardstick); "
                     "the headline c2 always runs, c2s adds its single-launch figure")
     ap.add_argument("--summarize", metavar="DIR", help="print a text summary of rocprofv3 CSV output and exit")
     args = ap.parse_args()
@@ -556,13 +553,6 @@ def main():
         msf = timed(lambda: o3.fill_(1.0), 20, 2, torch.cuda.current_stream())
         del o3
         extra["c3_output_write_alone"] = {"us": round(msf * 1e3, 2), "what": "torch fill_ of the 512 x 8192 fp32 output"}
-    if "c3" in only or "c3g" in only:
-        # the same ROW GEMM through the generic copy (every shape that is not c3's runs it)
-        ms3g, _ = gemm(20, 2, generic=True)
-        tops = 2 * 512 * 2048 * 8192 / (ms3g * 1e-3) / 1e12
-        extra["c3_gemm_row_x_rsc_generic_copy"] = {"us": round(ms3g * 1e3, 2), "TOPS": round(tops, 2),
-                                                   "frac_int8_peak": round(tops / INT8_PEAK_TOPS, 4)}
-        print(f"[c3 generic copy] {extra['c3_gemm_row_x_rsc_generic_copy']}", file=sys.stderr, flush=True)
     if "c3blas" in only:
         msb = int_mm(20, 2)
         tops = 2 * 512 * 2048 * 8192 / (msb * 1e-3) / 1e12

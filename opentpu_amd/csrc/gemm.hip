@@ -15,8 +15,6 @@
 // distinct banks); each of its 4 multiplying waves computes 64 x 64 with 4 x 4
 // v_mfma_i32_16x16x64_i8.  Tiles are assigned XCD-major: the workgroups of one XCD share weight
 // rows, so each weight panel is fetched from HBM once into that XCD's L2.
-#include <cstdlib>
-
 #include "prefill_impl.h"
 
 namespace otpu {
@@ -484,28 +482,24 @@ __device__ __forceinline__ void lw_mma_walk_h(const int8_t* ring, const uint32_t
 }
 #undef OTPU_READS_UNDER_MMA
 
-// C3: a copy for the c3 prefill shape (M 512, N 8192, K 2048, dense rows, RSC scale words), its
-// sizes and strides as constants (the kernel runs once a CU from a cold instruction cache)
-#ifndef OTPU_GEMM_C3
-#define OTPU_GEMM_C3 1
-#endif
-// The GEMM with loader waves (workgroups of 8 waves; C3: the c3 shape's copy).  Waves 0-3 scan the
+// The GEMM with loader waves (workgroups of 8 waves).  DENSE: whole tiles of dense rows (RSC words, float4 stores),
+// whose strides follow from the sizes: a tile runs once a round from a cold instruction cache, so the shorter
+// code is its latency (512 x 2048 x 8192 ROW 14.5 -> 14.05 us).  Waves 0-3 scan the
 // tile's offsets, multiply and store; waves 4-7 issue the ring's direct loads (and store half of a
 // full tile).  Tiles of one or two activation offsets walk the ring with both groups; any other
 // tile waits for the loaders' stages to land and takes the walk of any offsets (prefill_impl.h) on
 // all 8 waves.
-template <bool C3>
+template <bool DENSE>
 __global__ __launch_bounds__(512) void gemm_lw_kernel(GemmArgs a) {
-    if constexpr (C3) {
-        a.M = 512; a.N = 8192; a.K = 2048; a.ldq = 2048; a.rs = 2048; a.ldda = 64; a.srs = 4; a.ors = 8192;
-        a.tiles_m = 4; a.tiles_n = 64; a.vec4 = 1;
+    if constexpr (DENSE) {
+        a.ldq = a.rs = a.K; a.ldda = a.K / 32; a.srs = 4; a.ors = a.N; a.vec4 = 1;
     }
     __shared__ __align__(16) int8_t sRing[RING];
     __shared__ uint32_t sMask[4];
     __shared__ uint32_t sDaAll[GBM * DAS];
     __shared__ float sSa2[GBM];
 
-    const int tid = threadIdx.x, lane = tid & 63, wid = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int tid = threadIdx.x, wid = __builtin_amdgcn_readfirstlane(tid >> 6);
     const bool loader = wid >= 4;
     int b = blockIdx.x, tm, tn;
     const int ntiles = a.tiles_m * a.tiles_n;
@@ -527,7 +521,7 @@ __global__ __launch_bounds__(512) void gemm_lw_kernel(GemmArgs a) {
     // wave w and loader w + 4, region w & 3): a loader's before its ring loads, which complete
     // in order after them (the stage waits' counts unchanged), a compute wave's after the
     // offset scan (whose waits would otherwise wait for them too)
-    const bool split = m0 + GBM <= a.M && n0 + GBN <= a.N && a.vec4;
+    const bool split = DENSE || (m0 + GBM <= a.M && n0 + GBN <= a.N && a.vec4);
     float esw[4] = {1.0f, 1.0f, 1.0f, 1.0f};
     if (loader) {
         if (split) epi_sw(a, n0, wid & 3, esw);
@@ -639,11 +633,8 @@ int otpu_gemm_try(const int8_t* q, int64_t ldq, const float* Sa, const uint8_t* 
     a.tiles_m = (M + GBM - 1) / GBM;
     a.tiles_n = (N + GBN - 1) / GBN;
     a.vec4 = ((uintptr_t)out % 16 == 0) && (ors % 4 == 0);
-    // (OTPU_GENERIC_COPIES set: the generic copy for every shape, the same results; for measuring
-    // what the c3 copy is worth on the same operands)
-    const bool c3 = OTPU_GEMM_C3 && M == 512 && N == 8192 && K == 2048 && ldq == 2048 && rs == 2048 && ldda == 64 &&
-                    srs == 4 && ors == 8192 && a.vec4 && !getenv("OTPU_GENERIC_COPIES");
-    if (c3) gemm_lw_kernel<true><<<a.tiles_m * a.tiles_n, 512, 0, s>>>(a);
+    const bool dense = M % GBM == 0 && N % GBN == 0 && ldq == K && rs == K && ldda == K / 32 && srs == 4 && ors == N && a.vec4;
+    if (dense) gemm_lw_kernel<true><<<a.tiles_m * a.tiles_n, 512, 0, s>>>(a);
     else gemm_lw_kernel<false><<<a.tiles_m * a.tiles_n, 512, 0, s>>>(a);
     return otpu_launch_check("mm gemm");
 }
