@@ -248,12 +248,14 @@ def _overlap(a, b) -> bool:
     return pa < pb + b.numel() * b.element_size() and pb < pa + a.numel() * a.element_size()
 
 
-def _dot_row(x, w: QWeight, ranges, out) -> bool:
+def _dot_row(x, w: QWeight, ranges, out, given: bool) -> bool:
     """One fp32 row x (a contiguous device tensor [1, K]) @ w^T into out in one launch, QACT and the
-    ranges' ACC chain inside; False where no such kernel takes the call, or out overlaps x (every
-    workgroup reads the row while others store)."""
+    ranges' ACC chain inside; False where no such kernel takes the call, or out, where the caller gave
+    it, overlaps x (every workgroup reads the row while others store)."""
     K, width = w.K, ranges[0]
-    if min(ranges) != max(ranges) or x.data_ptr() % 16 or not _row_launch(w.fmt, w.N, K, width) or _overlap(x, out):
+    if len(ranges) > 1 and min(ranges) != max(ranges):
+        return False
+    if x.data_ptr() % 16 or not _row_launch(w.fmt, w.N, K, width) or (given and _overlap(x, out)):
         return False
     ws, srs = (0, 0) if w.srows is None else (w.srows.data_ptr(), w.srows.shape[1])
     fl = _flags(w.srows is None, w.rsc)
@@ -316,7 +318,7 @@ def dot(x, w: QWeight, acc=None, out=None, ranges=None, row_mode: bool = False, 
         ranges = _check_ranges(ranges, K)
         if M == 1 and not (row_mode or rowmax) and acc is None and acc_scale is None:
             y = out if out is not None else X.empty((1, N), np.float32)
-            if _dot_row(xd, w, ranges, y):
+            if _dot_row(xd, w, ranges, y, out is not None):
                 return X.host(y) if numpy_in else y
     else:
         q, Sa, da, ranges = x
