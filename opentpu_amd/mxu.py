@@ -209,12 +209,13 @@ def C_ptr(t, off: int):
 
 # One row's launches: QACT inside the GEMV (otpu_mm_qin, otpu_mm_qin_fold) saves a launch of ~3 us, and every
 # workgroup quantizes the whole row again.  So the columns they quantize together (otpu_qin_columns) decide.  Up
-# to 2.5M the single launch is the faster nearly everywhere (weight rows x columns, us, one / two launches: int4
-# 4096 x 1024 4.6 / 6.1, 6144 x 4096 (3.0M) 7.7 / 8.0, 16384 x 4096 14.3 / 11.4, 12288 x 16384 63 / 37; int8 4096 x
-# 4096 7.6 / 8.6, 12288 x 12288 59 / 39).  A fold of 256-column ranges: up to 8M (int4 1024 x 3072 5.8 / 10.5,
-# 8192 x 8192 28.8 / 24.8); of wider ones, whose sums a team's first lane adds one after another: up to 3M (2048
-# x 6144 11.4 / 11.5, 4096 x 6144 16.1 / 11.8).
-QIN_COLUMNS = 5 << 19
+# to 3M (2M past 16384 weight rows) the single launch is the faster nearly everywhere (weight rows x columns, us,
+# one / two launches: int4 4096 x 1024 4.6 / 6.1, 4096 x 6144 (3M) 8.3 / 9.3, 16384 x 4096 14.3 / 11.4, 12288 x 16384
+# 63 / 37; int8 4096 x 4096 7.6 / 8.6, 12288 x 12288 59 / 39).  A fold of 256-column ranges: up to 8M (int4 1024 x
+# 3072 5.8 / 10.5, 8192 x 8192 28.8 / 24.8); of wider ones, whose sums a team's first lane adds one after another: up
+# to 3M (2048 x 6144 11.4 / 11.5, 4096 x 6144 16.1 / 11.8).
+QIN_COLUMNS = 3 << 20
+TALL_QIN_COLUMNS = 2 << 20
 FOLD_COLUMNS = 8 << 20
 WIDE_FOLD_COLUMNS = 3 << 20
 OFF_COLS = 1 << 24                                        # otpu_mm_dot's rows: 32-bit offsets over a tile's rows
@@ -228,18 +229,20 @@ def _row_launch(fmt: str, N: int, K: int, width: int) -> bool:
         return 0 < cols <= (FOLD_COLUMNS if width == 256 else WIDE_FOLD_COLUMNS)
     # (int8 rows of eight pieces a lane: the kernel's prologue is compiled for 16384 columns and leaves one wave
     # a SIMD; 4096 x 8192 16.7 us against 11.7.  Past 8192 the other GEMV walks segments: 4096 x 10240 19.9 / 21.1)
-    return 0 < cols <= QIN_COLUMNS and not (fmt == "int8" and 6144 < K <= 8192)
+    return 0 < cols <= (QIN_COLUMNS if N <= 16384 else TALL_QIN_COLUMNS) and not (fmt == "int8" and 6144 < K <= 8192)
 
 
 # ... and in ranges: the GEMV of every range and the sum of their rows (otpu_mm_ranges) in place of otpu_mm_dot's
 # tiles of 16 and 32 rows, where those are mostly padding and weights enough stream by.  One row (us, GEMV / tiles,
 # QACT in): int4 12288 x 8192 18.6 / 29.7, 2048 x 8192 10.6 / 12.7, 4096 x 1024 8.8 / 7.4; int8 2048 x 16384 13.9 /
-# 19.4, 2048 x 2048 9.7 / 8.5.  Two (without QACT): int4 12288 x 2048 12.2 / 16.9, 8192 x 2048 10.9 / 7.8.  Four: 70000
-# x 1024 int4 39.9 / 45.3, int8 34.0 / 29.0.
+# 19.4, 16384 x 8192 35.7 / 29.6.  Two (without QACT): int4 12288 x 2048 12.2 / 16.9, 8192 x 2048 10.9 / 7.8; int8 20000 x
+# 1024 10.5 / 13.9.  Four: 70000 x 1024 int4 39.9 / 45.3, int8 34.0 / 29.0.
 def _stream_ranges(M: int, N: int, fmt: str, width: int) -> bool:
+    if fmt == "int8":
+        return M <= 2 and (N >= 20000 or (M == 1 and width >= 1280))
     if M <= 2:
         return N >= 12288 or (M == 1 and width >= 512)
-    return M <= 4 and fmt != "int8" and N >= 24576
+    return M <= 4 and N >= 24576
 
 
 def _overlap(a, b) -> bool:

@@ -100,13 +100,16 @@ def names(calls):
     ("int4", 64, 8448, 256, ["qact_ranges", "mm_dot"]), ("int4", 64, 8448, 768, ["qact_ranges", "mm_ranges"]),
     ("int4", 2048, 6144, 768, ["mm_qin_fold"]), ("int4", 4096, 6144, 768, ["qact_ranges", "mm_ranges"]),
     ("int4", 64, 1024, 128, ["qact_ranges"] + ["mm"] * 8), ("int8", 64, 1024, 128, ["qact_ranges", "mm_dot"]),
-    ("int8", 12288, 512, 256, ["qact_ranges", "mm_ranges"]), ("int8", 12287, 512, 256, ["qact_ranges", "mm_dot"])])
+    ("int4", 4096, 6144, None, ["mm_qin"]), ("int4", 4104, 6144, None, ["qact", "mm_dot"]),
+    ("int4", 20000, 2048, None, ["mm_qin"]), ("int4", 32800, 2048, None, ["qact", "mm_dot"]),
+    ("int8", 64, 10240, 1280, ["qact_ranges", "mm_ranges"]), ("int8", 64, 8192, 1024, ["qact_ranges", "mm_dot"]),
+    ("int8", 20000, 512, 256, ["qact_ranges", "mm_ranges"]), ("int8", 19999, 512, 256, ["qact_ranges", "mm_dot"])])
 def test_one_rows_launches(calls, fmt, N, K, width, want):
     mxu.dot(torch.zeros((1, K)), weight(N, K, fmt), ranges=None if width is None else [width] * (K // width))
     assert names(calls) == want
 
 
-@pytest.mark.parametrize("M,fmt,N,want", [(2, "int4", 12287, "mm_dot"), (2, "int8", 12288, "mm_ranges"), (3, "int4", 12288, "mm_dot"),
+@pytest.mark.parametrize("M,fmt,N,want", [(2, "int4", 12287, "mm_dot"), (2, "int8", 20000, "mm_ranges"), (2, "int8", 19999, "mm_dot"), (3, "int4", 12288, "mm_dot"),
                                           (4, "nvfp4", 24576, "mm_ranges"), (4, "int8", 24576, "mm_dot"), (5, "int4", 24576, "mm_dot")])
 def test_few_rows_launches_in_ranges(calls, M, fmt, N, want):
     w = weight(N, 512, fmt)

@@ -142,9 +142,9 @@ def dot64(x, rows, srows, fmt, K, widths, old=None, row_mode=False):
     return want
 
 
-ONE = [(40, 256, None), (40, 384, None), (16384, 512, None), (16385, 512, None), (40, 6144, None), (40, 6400, None), (40, 8192, None),
-       (40, 8448, None), (70, 16384, None), (70, 16640, None), (2300, 4096, None), (6000, 4096, None),
-       (12287, 512, 256), (12288, 512, 256), (30, 8192, 256), (30, 8448, 256), (30, 8448, 768), (4096, 6144, 768), (50, 1024, 128),
+ONE = [(40, 256, None), (40, 384, None), (20000, 2048, None), (32800, 2048, None), (40, 6144, None), (40, 6400, None), (40, 8192, None),
+       (40, 8448, None), (70, 16384, None), (70, 16640, None), (4096, 6144, None), (4104, 6144, None),
+       (12287, 512, 256), (12288, 512, 256), (20000, 512, 256), (60, 10240, 1280), (30, 8192, 256), (30, 8448, 256), (30, 8448, 768), (4096, 6144, 768), (50, 1024, 128),
        (50, 1024, (512, 256, 256)), (50, 1024, (256, 512, 256))]
 
 
@@ -166,7 +166,7 @@ def test_one_row_at_the_rules_edges(mxu, fmt):
         assert same_bits(got, np.resize(want[0], (1, N))), (N, K, width)
 
 
-@pytest.mark.parametrize("M,fmt,N", [(1, "int8", 12288), (2, "int4", 12288), (2, "rsc", 12300), (3, "nvfp4", 24576), (4, "fp4", 24600),
+@pytest.mark.parametrize("M,fmt,N", [(1, "int8", 20000), (2, "int4", 12288), (2, "rsc", 20003), (3, "nvfp4", 24576), (4, "fp4", 24600),
                                      (4, "int4", 24575)])
 def test_few_rows_on_many_weights_in_ranges(mxu, M, fmt, N):
     """The GEMV of every range and the sum of their rows: overwriting, onto old values, from an operand."""
@@ -185,3 +185,37 @@ def test_few_rows_on_many_weights_in_ranges(mxu, M, fmt, N):
     assert same_bits(mxu.dot(mxu.quantize_ranges(xd, [width] * 3), w).cpu().numpy(), want)
     acc = torch.from_numpy(np.ascontiguousarray(old[:, idx])).cuda()
     assert same_bits(mxu.dot(xd, w, acc=acc, ranges=[width] * 3).cpu().numpy(), dot64(x, rows, srows, fmt, K, [width] * 3, old)[:, idx])
+
+
+def test_dots_under_capture(mxu):
+    """One dot of each route in a graph: replays on new rows with eager work between, and on another stream."""
+    import torch
+    rng = np.random.default_rng(9)
+    calls = []
+    for fmt, M, N, K, width in (("int4", 1, 256, 1024, 1024), ("int4", 1, 256, 3072, 256), ("int8", 1, 20000, 512, 256),
+                                ("nvfp4", 2, 12288, 512, 256), ("fp4", 6, 300, 512, 256), ("rsc", 130, 8200, 256, 256)):
+        rows, srows = packed(rng, 50, K, fmt)
+        w = qweight(mxu, np.resize(rows, (N, rows.shape[1])), np.resize(srows, (N, srows.shape[1])), fmt, K)
+        calls.append((torch.zeros((M, K), device="cuda"), w, [width] * (K // width)))
+    run = lambda: [mxu.dot(x, w, ranges=r) for x, w, r in calls]  # noqa: E731
+    run()
+    torch.cuda.synchronize()
+    g = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(g):
+        outs = run()
+    say("dots under capture")
+    side = torch.cuda.Stream()
+    for i in range(4):
+        for x, _, _ in calls:
+            x.copy_(torch.from_numpy(spread(rng, *x.shape, 2.0, 32)))
+        eager = [t.cpu().numpy() for t in run()]
+        torch.cuda.synchronize()
+        with torch.cuda.stream(side if i % 2 else torch.cuda.current_stream()):
+            g.replay()
+            torch.cuda.synchronize()
+        for a, b in zip(outs, eager):
+            assert same_bits(a.cpu().numpy(), b), i
+    with torch.cuda.stream(side):                         # eager on a stream of its own
+        again = run()
+    side.synchronize()
+    assert all(same_bits(a.cpu().numpy(), b) for a, b in zip(again, eager))
