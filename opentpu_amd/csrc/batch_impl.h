@@ -1,5 +1,6 @@
-// MM for a batch of activation rows (M >= 5) on the int8 MFMA units with the group scales applied
-// to the products, not folded into the operands.  Semantics: opentpu/isasim.py:749-910
+// MM for a batch of activation rows (more than four, or any number in several ranges: mm_rows in
+// gemv.hip) on the int8 MFMA units with the group scales applied to the products, not folded into the
+// operands.  Semantics: opentpu/isasim.py:749-910
 // (docs/isa.md:226-305), and the ranges' ACC chain of Builder.dot (opentpu/compiler.py:2686-2720).
 //
 // One v_mfma_i32_16x16x32_i8 is one 32-group of 16 activation rows x 16 weight rows: its int32 sums

@@ -328,7 +328,7 @@ __device__ __forceinline__ void lw_load_walk(const RingSrc& rs, int KS, int rot)
 }
 
 // a compute wave's walk: NP planes into acc[p]; MASK: each stage's A fragments masked to plane
-// p's 32-groups (plain weights, offsets from da_lds as in gemm_pass_mp), else the single plane.
+// p's 32-groups (plain weights, offsets from da_lds), else the single plane.
 // ALL1 (two planes covering every group): plane 1's product taken over every group instead,
 // C_all, so that only plane 0 is masked (C_1 = C_all - C_0 afterwards, exactly in int32).
 // KS + 1 barriers, matching lw_load_walk's.
