@@ -236,7 +236,11 @@ def _row_launch(fmt: str, N: int, K: int, width: int) -> bool:
 # tiles of 16 and 32 rows, where those are mostly padding and weights enough stream by.  One row (us, GEMV / tiles,
 # QACT in): int4 12288 x 8192 18.6 / 29.7, 2048 x 8192 10.6 / 12.7, 4096 x 1024 8.8 / 7.4; int8 2048 x 16384 13.9 /
 # 19.4, 16384 x 8192 35.7 / 29.6.  Two (without QACT): int4 12288 x 2048 12.2 / 16.9, 8192 x 2048 10.9 / 7.8; int8 20000 x
-# 1024 10.5 / 13.9.  Four: 70000 x 1024 int4 39.9 / 45.3, int8 34.0 / 29.0.
+# 1024 10.5 / 13.9.  Four: 70000 x 1024 int4 39.9 / 45.3, int8 34.0 / 29.0.  It takes a workspace of a row a range, so
+# not where that is large.
+PART_BYTES = 1 << 28
+
+
 def _stream_ranges(M: int, N: int, fmt: str, width: int) -> bool:
     if fmt == "int8":
         return M <= 2 and (N >= 20000 or (M == 1 and width >= 1280))
@@ -343,7 +347,8 @@ def dot(x, w: QWeight, acc=None, out=None, ranges=None, row_mode: bool = False, 
     if one:
         s = X.stream()
         R = len(ranges)
-        stream = R > 1 and al is None and R < 1 << 16 and _stream_ranges(M, N, w.fmt, width)
+        stream = (R > 1 and al is None and R < 1 << 16 and 4 * R * M * N <= PART_BYTES
+                  and _stream_ranges(M, N, w.fmt, width))
         sizes = (4 * R * M * N,) if stream else ()
         if operand:
             qp, Sp, dp, act = q.data_ptr(), Sa[0].data_ptr(), da.data_ptr(), _operand_act(x, w)

@@ -137,3 +137,11 @@ def test_an_operands_mode_picks_the_kernel(calls, fmt):
             calls.clear()
             mxu.dot(x, w)
             assert names(calls) == ["mm_dot"] and calls[0][17] == act
+
+
+@pytest.mark.parametrize("K,want", [(1 << 19, "mm_ranges"), (3 << 19, "mm_dot")])
+def test_a_workspace_of_ranges_is_bounded(calls, K, want):
+    """A row a range of fp32 for one row on 20000 weight rows: 164 MB over 2048 ranges, 492 MB over 6144."""
+    w = mxu.QWeight(torch.empty((20000, 1), dtype=torch.uint8), torch.empty((20000, 1), dtype=torch.uint8), "int4", K)
+    mxu.dot(torch.empty((1, K)), w, ranges=[256] * (K // 256))
+    assert names(calls) == ["qact_ranges", want]

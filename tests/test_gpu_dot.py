@@ -128,7 +128,7 @@ def test_ranges_over_a_part_of_an_operand(mxu, fmt, M):
             assert same_bits(mxu.dot((q, S, da, [256] * R), w).cpu().numpy(), want)
 
 
-def dot64(x, rows, srows, fmt, K, widths, old=None, row_mode=False):
+def oracle_dot(x, rows, srows, fmt, K, widths, old=None, row_mode=False):
     """The oracle's dot: a QACT and an MM a range, the MMs' outputs added in range order."""
     want, c0 = old, 0
     bpb = 128 if fmt in ("int8", "rsc") else 64
@@ -162,7 +162,7 @@ def test_one_row_at_the_rules_edges(mxu, fmt):
         x = spread(rng, 1, K, 2.0, 32)
         say("one row", fmt, N, K, width)
         got = mxu.dot(torch.from_numpy(x).cuda(), qweight(mxu, rows, srows, fmt, K), ranges=widths).cpu().numpy()
-        want = dot64(x, np.ascontiguousarray(rows[:some]), np.ascontiguousarray(srows[:some]), fmt, K, widths)
+        want = oracle_dot(x, np.ascontiguousarray(rows[:some]), np.ascontiguousarray(srows[:some]), fmt, K, widths)
         assert same_bits(got, np.resize(want[0], (1, N))), (N, K, width)
 
 
@@ -180,11 +180,11 @@ def test_few_rows_on_many_weights_in_ranges(mxu, M, fmt, N):
     old = np.resize(rng.standard_normal((M, some)).astype(np.float32), (M, some))
     idx = np.arange(N) % some
     say("few rows", M, fmt, N)
-    want = dot64(x, rows, srows, fmt, K, [width] * 3)[:, idx]
+    want = oracle_dot(x, rows, srows, fmt, K, [width] * 3)[:, idx]
     assert same_bits(mxu.dot(xd, w, ranges=[width] * 3).cpu().numpy(), want)
     assert same_bits(mxu.dot(mxu.quantize_ranges(xd, [width] * 3), w).cpu().numpy(), want)
     acc = torch.from_numpy(np.ascontiguousarray(old[:, idx])).cuda()
-    assert same_bits(mxu.dot(xd, w, acc=acc, ranges=[width] * 3).cpu().numpy(), dot64(x, rows, srows, fmt, K, [width] * 3, old)[:, idx])
+    assert same_bits(mxu.dot(xd, w, acc=acc, ranges=[width] * 3).cpu().numpy(), oracle_dot(x, rows, srows, fmt, K, [width] * 3, old)[:, idx])
 
 
 def test_dots_under_capture(mxu):
