@@ -209,12 +209,32 @@ static bool gemm_pays(int M, int N, int K, int fmt, bool plain) {
     return gemm < c.start + c.start_k * kb + tiles * (c.tile + c.tile_k * kb);
 }
 
+// 5 to 8 activation rows on 4-bit weights: does the GEMV, its rows in two passes, pay?  The time of the batch and
+// prefill kernels goes by steps, a round of their tiles (or a half) at a time, the GEMV's by weight rows, so it pays
+// where a step has just begun and few lanes are idle.  GEMV / the better of the two, K = 2048 and 4096, by
+// 128-row tiles of weights a CU (CUs = 256):
+//   5 and 6 rows, 17/32 to 5/8: int4 .81 to .95, fp4 .84 to .97; 1+ to 5/4: .72 to .86, .81 to 1.02; between them
+//     (3/4 to 15/16) .98 to 1.28, past them (7/4 to 2) .93 to 1.52
+//   nvfp4, whose weights these kernels unpack more slowly: 9/32 to 7/16 .72 to 1.00, 17/32 to 13/8 .61 to 1.04, past
+//     it .92 to 1.34; 7 and 8 rows .78 to .88 and .81 to 1.01 in the two windows (int4 and fp4 .92 to 1.25); K = 512,
+//     1024 and 6144, whose lanes are all busy, .80 to 1.01 there (768 and 1536 .94 to 1.19, 8192 .88 to 1.08)
+static bool gemv_pays(int M, int N, int K, int fmt) {
+    if (M > 8 || fmt == OTPU_INT8) return false;
+    const int64_t n = (N + 127) / 128, cus = otpu_cu_count();
+    const bool begun = (n > cus / 2 && n <= cus * 5 / 8) || (n > cus && n <= cus * 5 / 4);
+    int T, L;
+    pick_team(K / 32, &T, &L);
+    const bool best = T == 64 && L <= 2 && (T * L * 32 - K) * 16 <= K;
+    if (fmt != OTPU_NVFP4) return best && begun && M <= 6;
+    if (best && M <= 6) return (n > cus / 4 && n <= cus * 7 / 16) || (n > cus / 2 && n <= cus * 13 / 8);
+    return begun && (best || (M <= 6 && T * L * 32 == K && (L == 1 || (L == 3 && T == 64))));
+}
+
 // MM of several activation rows, over `ranges` equal column ranges (their ACC chain): 0 or an error, or > 0
 // where none of these kernels takes the call (RMAX, offset rows that are not whole words: the GEMV then
 // streams it, a few rows a launch).  act: what is known of the activation offsets (OTPU_ACT_*).  The kernels
 // give the same bits; the lines between them, measured (M x K x N, us):
-//   the GEMV, its rows in two passes, for 5 and 6 rows on many 4-bit weights of one or two pieces a lane: int4 5 x
-//     4096 x 40000 38 against 48 (batch) and 56 (prefill), 6 x 2048 x 28672 21 / 18 / 24, nvfp4 5 x 2048 x 20000 21 / 28
+//   the GEMV, its rows in two passes, for 5 to 8 rows of 4-bit weights where it pays (above)
 //   the batch kernel (no LDS; K split over waves) below 9/16 of a 32 x 128 tile a CU, 3/4 for up to 16 rows:
 //     batch / prefill int4 64 x 2048 x 8192 (128 tiles) 17.5 / 22.7, 300 x 6144 x 2048 (160) 60 / 56, int8 33 x 8192 x
 //     8192 (128) 38 / 70, nvfp4 32 x 1024 x 20000 (157) 28.9 / 18.6; plain int8 16 x 1024 x 20000 13.5 / 9.8, and with one
@@ -230,14 +250,10 @@ static int mm_rows(const int8_t* q, int64_t ldq, const float* Sa, const uint8_t*
     if (flags & OTPU_RMAX) return 1;
     const bool plain = (flags & (OTPU_UNIT | OTPU_RSC)) != 0, int8 = fmt == OTPU_INT8;
     const int64_t n128 = (N + 127) / 128, cus = otpu_cu_count();
-    if (ranges == 1 && M <= 6 && !int8 && K >= 2048 && n128 >= cus * 9 / 16 && n128 <= cus * 5 / 2) {
-        int T, L;
-        pick_team(K / 32, &T, &L);
-        if (L <= 2) {
-            MMArgs a = make_args(q, ldq, Sa, da, ldda, M, K, w, rs, ws, srs, N, flags, k0);
-            a.alpha = alpha; a.out = out; a.ors = ors;
-            return launch_gemv(a, fmt, 1, s);
-        }
+    if (ranges == 1 && gemv_pays(M, N, K, fmt)) {
+        MMArgs a = make_args(q, ldq, Sa, da, ldda, M, K, w, rs, ws, srs, N, flags, k0);
+        a.alpha = alpha; a.out = out; a.ors = ors;
+        return launch_gemv(a, fmt, 1, s);
     }
     const bool plain8 = int8 && plain && ranges == 1;
     const int64_t sixteenths = M <= 16 ? (plain8 ? 9 : 12) : plain8 && act == OTPU_ACT_ROW ? 5 : 9;

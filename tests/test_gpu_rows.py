@@ -134,7 +134,9 @@ def test_gemm_kinds(X, M0, N0, K, fmt, wk, ak, k0):
         assert same_bits(got, OC.mm(q, Sa, da, rows, srows, fmt, K, flags=fl | MM.ACC, k0=k0, old=old)[:, idx])
 
 
-@pytest.mark.parametrize("M,N,K", [(5, 18305, 2048), (6, 18304, 4096), (7, 18305, 2048), (5, 18305, 2304), (16, 20000, 256), (17, 18400, 256)])
+@pytest.mark.parametrize("M,N,K", [(5, 18305, 2048), (6, 20480, 4096), (7, 18305, 2048), (5, 18305, 2304), (16, 20000, 256), (17, 18400, 256),
+                                   (8, 20481, 4096), (6, 32769, 2048), (8, 32770, 2048), (6, 8193, 4096), (5, 8192, 4096), (5, 18305, 512),
+                                   (6, 18305, 1024), (5, 18305, 6144)])
 @pytest.mark.parametrize("fmt,wk,ak", [("int8", "rsc", "mx"), ("int8", "spread", "mx"), ("int4", "x4", "mx"), ("nvfp4", "x4", WIN)])
 def test_few_rows_on_many_weights(X, M, N, K, fmt, wk, ak):
     """Both sides of the lines between the GEMV, the batch and the prefill kernel, onto old values."""
