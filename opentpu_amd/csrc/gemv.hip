@@ -213,21 +213,47 @@ static bool gemm_pays(int M, int N, int K, int fmt, bool plain) {
 // prefill kernels goes by steps, a round of their tiles (or a half) at a time, the GEMV's by weight rows, so it pays
 // where a step has just begun and few lanes are idle.  GEMV / the better of the two, K = 2048 and 4096, by
 // 128-row tiles of weights a CU (CUs = 256):
-//   5 and 6 rows, 17/32 to 5/8: int4 .81 to .95, fp4 .84 to .97; 1+ to 5/4: .72 to .86, .81 to 1.02; between them
-//     (3/4 to 15/16) .98 to 1.28, past them (7/4 to 2) .93 to 1.52
-//   nvfp4, whose weights these kernels unpack more slowly: 9/32 to 7/16 .72 to 1.00, 17/32 to 13/8 .61 to 1.04, past
-//     it .92 to 1.34; 7 and 8 rows .78 to .88 and .81 to 1.01 in the two windows (int4 and fp4 .92 to 1.25); K = 512,
-//     1024 and 6144, whose lanes are all busy, .80 to 1.01 there (768 and 1536 .94 to 1.19, 8192 .88 to 1.08)
+//   5 and 6 rows, 1/2+ to 5/8: int4 .81 to .95, fp4 .84 to .97; 1+ to 5/4: .72 to .86 (to 11/8 .91), .81 to 1.02;
+//     between them (3/4 to 15/16) .98 to 1.28, past them (7/4 to 2) .93 to 1.52; int4, K = 512 .83 to .91 and .94 to
+//     1.00, K = 1024 1.05 to 1.11 and .87 to 1.01
+//   nvfp4, whose weights these kernels unpack more slowly: 1/4+ to 7/16 .72 to 1.00, 1/2+ to 13/8 .61 to 1.04, past it
+//     .92 to 1.34; 7 and 8 rows, 1/4+ to 5/16 .86 to .89 (3/8 .99 to 1.02), the two windows .78 to .88 and .81 to 1.01
+//     (int4 and fp4 .92 to 1.25); K = 512, 1024 and 6144, whose lanes are all busy, .80 to 1.01 there (768 and 1536
+//     .94 to 1.19, 8192 .88 to 1.08)
 static bool gemv_pays(int M, int N, int K, int fmt) {
     if (M > 8 || fmt == OTPU_INT8) return false;
     const int64_t n = (N + 127) / 128, cus = otpu_cu_count();
-    const bool begun = (n > cus / 2 && n <= cus * 5 / 8) || (n > cus && n <= cus * 5 / 4);
+    const bool first = n > cus / 2 && n <= cus * 5 / 8, second = n > cus && n <= cus * 5 / 4;
     int T, L;
     pick_team(K / 32, &T, &L);
-    const bool best = T == 64 && L <= 2 && (T * L * 32 - K) * 16 <= K;
-    if (fmt != OTPU_NVFP4) return best && begun && M <= 6;
-    if (best && M <= 6) return (n > cus / 4 && n <= cus * 7 / 16) || (n > cus / 2 && n <= cus * 13 / 8);
-    return begun && (best || (M <= 6 && T * L * 32 == K && (L == 1 || (L == 3 && T == 64))));
+    const bool best = T == 64 && L <= 2 && (T * L * 32 - K) * 16 <= K, full = T * L * 32 == K;
+    if (fmt == OTPU_INT4 && M <= 6)
+        return best ? first || (n > cus && n <= cus * 11 / 8) : full && L == 1 && (second || (first && T == 16));
+    if (fmt != OTPU_NVFP4) return M <= 6 && best && (first || second);
+    if (best && n > cus / 4 && n <= (M <= 6 ? cus * 7 / 16 : cus * 5 / 16)) return true;
+    if (best && M <= 6) return n > cus / 2 && n <= cus * 13 / 8;
+    return (first || second) && (best || (M <= 6 && full && (L == 1 || (L == 3 && T == 64))));
+}
+
+// Does the batch kernel (no LDS; K split over waves) pay, beside the prefill kernel and the GEMMs?  n: 128-row tiles
+// of weights; batch / prefill, at 256 CUs.
+//   more than 16 rows, or ranges: below 9/16 of a 32 x 128 tile a CU (3/4 for up to 16 rows): us, int4 64 x 2048 x
+//     8192 (128 tiles) 17.5 / 22.7, 300 x 6144 x 2048 (160) 60 / 56, int8 33 x 8192 x 8192 (128) 38 / 70, nvfp4 32 x
+//     1024 x 20000 (157) 28.9 / 18.6; plain int8 with one offset, where the GEMM starts sooner, below 5/16: 384 x 2048
+//     x 1024 (96) 16.3 / 12.3
+//   up to 16 rows, one range: its time goes by steps of half a tile a CU.  The first pays (.34 to .96, plain int8 to
+//     1.12; K = 256 .85 to 1.24).  The second, to 15/16, pays from K = 1024 (int4 .60 to .94, fp4 .75 to 1.08, int8 .66
+//     to 1.02, nvfp4 .87 to 1.01, but 1.08 to 1.19 at K = 1536, which its 8 waves share unevenly), not below it (.95 to
+//     1.8) nor for plain int8 (1.00 to 1.32), and full (256) for int4 alone from K = 3072 (.79 to .94), which has the
+//     third as well (.81 to .98; the fourth 1.12 to 1.26)
+static bool batch_pays(int M, int N, int K, int ranges, int fmt, bool plain8, int act) {
+    const int64_t n = (N + 127) / 128, cus = otpu_cu_count();
+    if (M > 16) return (M + 31) / 32 * n < cus * (plain8 && act == OTPU_ACT_ROW ? 5 : 9) / 16;
+    if (ranges > 1) return n < cus * 3 / 4;
+    if (n <= cus / 2) return true;
+    if (plain8 || K < 1024) return false;
+    if (fmt == OTPU_INT4 && K >= 3072) return n <= cus * 3 / 2;
+    return n <= cus * 15 / 16 && (fmt != OTPU_NVFP4 || K % 1024 == 0 || K >= 3072);
 }
 
 // MM of several activation rows, over `ranges` equal column ranges (their ACC chain): 0 or an error, or > 0
@@ -235,10 +261,7 @@ static bool gemv_pays(int M, int N, int K, int fmt) {
 // streams it, a few rows a launch).  act: what is known of the activation offsets (OTPU_ACT_*).  The kernels
 // give the same bits; the lines between them, measured (M x K x N, us):
 //   the GEMV, its rows in two passes, for 5 to 8 rows of 4-bit weights where it pays (above)
-//   the batch kernel (no LDS; K split over waves) below 9/16 of a 32 x 128 tile a CU, 3/4 for up to 16 rows:
-//     batch / prefill int4 64 x 2048 x 8192 (128 tiles) 17.5 / 22.7, 300 x 6144 x 2048 (160) 60 / 56, int8 33 x 8192 x
-//     8192 (128) 38 / 70, nvfp4 32 x 1024 x 20000 (157) 28.9 / 18.6; plain int8 16 x 1024 x 20000 13.5 / 9.8, and with one
-//     offset, where the GEMM starts sooner, below 5/16: 384 x 2048 x 1024 (96) 16.3 / 12.3
+//   the batch kernel where it pays (above)
 //   the GEMM for plain int8 and 4-bit weights: with one activation offset (ROW) where it pays (above); with several
 //     it is the slower (int4 4096 x 2048 x 8192 376 / 295; two offsets of plain int8 alone are the faster there, by
 //     up to 1.5, and three the slower by up to 1.3); with offsets unknown where it would pay and its last round of
@@ -256,8 +279,7 @@ static int mm_rows(const int8_t* q, int64_t ldq, const float* Sa, const uint8_t*
         return launch_gemv(a, fmt, 1, s);
     }
     const bool plain8 = int8 && plain && ranges == 1;
-    const int64_t sixteenths = M <= 16 ? (plain8 ? 9 : 12) : plain8 && act == OTPU_ACT_ROW ? 5 : 9;
-    if ((M + 31) / 32 * n128 < cus * sixteenths / 16)
+    if (batch_pays(M, N, K, ranges, fmt, plain8, act))
         return otpu_batch_try(q, ldq, Sa, da, ldda, M, K, ranges, w, rs, ws, srs, N, fmt, flags, k0, alpha, out, ors, s);
     if (ranges == 1 && (!int8 || plain) && act != OTPU_ACT_MX && gemm_pays(M, N, K, fmt, plain) &&
         (act == OTPU_ACT_ROW || (M + 127) / 128 * n128 * 5 / 4 >= pf::rounds(M, N, 128) * cus)) {

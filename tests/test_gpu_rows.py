@@ -136,7 +136,8 @@ def test_gemm_kinds(X, M0, N0, K, fmt, wk, ak, k0):
 
 @pytest.mark.parametrize("M,N,K", [(5, 18305, 2048), (6, 20480, 4096), (7, 18305, 2048), (5, 18305, 2304), (16, 20000, 256), (17, 18400, 256),
                                    (8, 20481, 4096), (6, 32769, 2048), (8, 32770, 2048), (6, 8193, 4096), (5, 8192, 4096), (5, 18305, 512),
-                                   (6, 18305, 1024), (5, 18305, 6144)])
+                                   (6, 18305, 1024), (5, 18305, 6144), (16, 30720, 1024), (9, 30721, 1024), (16, 16385, 1536), (10, 49152, 3072),
+                                   (6, 45056, 2048), (8, 10240, 2048), (6, 32900, 1024)])
 @pytest.mark.parametrize("fmt,wk,ak", [("int8", "rsc", "mx"), ("int8", "spread", "mx"), ("int4", "x4", "mx"), ("nvfp4", "x4", WIN)])
 def test_few_rows_on_many_weights(X, M, N, K, fmt, wk, ak):
     """Both sides of the lines between the GEMV, the batch and the prefill kernel, onto old values."""
